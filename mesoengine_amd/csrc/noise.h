@@ -125,18 +125,12 @@ __device__ __forceinline__ uint16_t height_band(int32_t y, int32_t n) {
   int32_t b = (y * 16) / n;
   return (uint16_t)(1 + (b < 3 ? b : 3));
 }
-__device__ __forceinline__ uint16_t terrain_caves_voxel(int32_t x, int32_t y, int32_t z,
-                                                        int32_t n, uint32_t seed, int32_t h) {
-  if (y >= h) return 0;
-  float c = fbm3((float)x, (float)y, (float)z, 3, 8.0f / (float)n, seed ^ 0x5bd1e995u);
-  c = c - 0.5f;
-  if (__builtin_fabsf(c) < 0.03f) return 0;
-  return height_band(y, n);
-}
-__device__ __forceinline__ uint16_t caves_voxel(int32_t x, int32_t y, int32_t z, uint32_t seed) {
-  float c = fbm3((float)x, (float)y, (float)z, 4, 1.0f / 64.0f, seed);
-  c = c - 0.5f;
-  if (__builtin_fabsf(c) >= 0.0055f) return 0;
+// Terrain voxels (three octaves of fbm3 of period n/8, seed ^ 0x5bd1e995) are
+// carved where the noise lies within kTunnelBand of 1/2; cave voxels (four
+// octaves of period 64) are solid where it lies within kCavesBand of 1/2.
+constexpr float kTunnelBand = 0.03f;
+constexpr float kCavesBand = 0.0055f;
+__device__ __forceinline__ uint16_t caves_material(int32_t y) {
   return (uint16_t)(1 + ((uint32_t)y >> 7) % 4u);
 }
 

@@ -2,6 +2,7 @@
 // two-level layouts, the chunk batch for meshing, the reference sphere
 // generator with its erosion mip chain, and brick edits.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <vector>
 
@@ -50,34 +51,30 @@ __global__ void scan_add_kernel(uint32_t *out, uint64_t n, const uint32_t *offse
     if (i + k < n) out[i + k] += add;
 }
 
-// out[i] = sum(in[0..i)); returns the total through *total_host.
-static meso_status scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, uint64_t *total_host,
-                            hipStream_t stream) {
-  if (n == 0) {
-    *total_host = 0;
-    return MESO_OK;
+// Workspace of scan_u32 over n elements: two words per 1024 elements and level.
+static uint64_t scan_ws_words(uint64_t n) {
+  uint64_t w = 0;
+  while (n > 1) {
+    n = (n + 1023) / 1024;
+    w += 2 * n;
   }
+  return w + 2;
+}
+
+// out[i] = sum(in[0..i)); the total goes to *total (device).  ws:
+// scan_ws_words(n) words; no allocation and no wait.
+static meso_status scan_u32(const uint32_t *in, uint32_t *out, uint64_t n, uint32_t *total,
+                            uint32_t *ws, hipStream_t stream) {
   const uint64_t nb = (n + 1023) / 1024;
-  uint32_t *sums = nullptr, *sums_scan = nullptr;
-  MESO_HIP(hipMallocAsync((void **)&sums, nb * 4, stream));
-  MESO_HIP(hipMallocAsync((void **)&sums_scan, nb * 4, stream));
+  uint32_t *sums = nb > 1 ? ws : total, *sums_scan = ws + nb;
   hipLaunchKernelGGL(scan_block_kernel, dim3((uint32_t)nb), dim3(256), 0, stream, in, out, n, sums);
   MESO_HIP(hipGetLastError());
-  uint64_t total = 0;
   if (nb > 1) {
-    meso_status st = scan_u32(sums, sums_scan, nb, &total, stream);
+    meso_status st = scan_u32(sums, sums_scan, nb, total, ws + 2 * nb, stream);
     if (st != MESO_OK) return st;
     hipLaunchKernelGGL(scan_add_kernel, dim3((uint32_t)nb), dim3(256), 0, stream, out, n, sums_scan);
     MESO_HIP(hipGetLastError());
-  } else {
-    uint32_t t = 0;
-    MESO_HIP(hipMemcpyAsync(&t, sums, 4, hipMemcpyDeviceToHost, stream));
-    MESO_HIP(hipStreamSynchronize(stream));
-    total = t;
   }
-  MESO_HIP(hipFreeAsync(sums, stream));
-  MESO_HIP(hipFreeAsync(sums_scan, stream));
-  *total_host = total;
   return MESO_OK;
 }
 
@@ -130,18 +127,6 @@ __global__ void heights_kernel(int32_t *h, int32_t n, uint32_t seed, int32_t gen
                                      : terrain_height(x, z, n, seed);
 }
 
-// One workgroup of 512 lanes per brick: wave w holds local z = w and lane
-// l = x + 8y, so the wave's ballot is exactly the brick's mask word z.
-__device__ __forceinline__ uint16_t gen_voxel(int32_t gen, int32_t x, int32_t y, int32_t z,
-                                              int32_t n, uint32_t seed, const int32_t *heights) {
-  if (gen == MESO_GEN_HEIGHTFIELD) {
-    return y < heights[(int64_t)z * n + x] ? height_band(y, n) : (uint16_t)0;
-  } else if (gen == MESO_GEN_TERRAIN_CAVES) {
-    return terrain_caves_voxel(x, y, z, n, seed, heights[(int64_t)z * n + x]);
-  }
-  return caves_voxel(x, y, z, seed);
-}
-
 // brick order: linear (brick map) or node-major (two-level: node * 4096 + local)
 __device__ __forceinline__ void brick_of(uint64_t ordered, int32_t nb, bool two_level, int32_t &bx,
                                          int32_t &by, int32_t &bz) {
@@ -161,58 +146,217 @@ __device__ __forceinline__ void brick_of(uint64_t ordered, int32_t nb, bool two_
   }
 }
 
-__global__ void __launch_bounds__(512) brick_flags_kernel(int32_t gen, int32_t n, uint32_t seed,
-                                                          const int32_t *heights, int32_t two_level,
-                                                          uint32_t *flags,
-                                                          unsigned long long *solid,
-                                                          uint64_t n_bricks) {
-  const uint64_t bid = block_id();
-  if (bid >= n_bricks) return;  // uniform over the workgroup
-  const int32_t nb = n / 8;
-  int32_t bx, by, bz;
-  brick_of(bid, nb, two_level != 0, bx, by, bz);
-  const int32_t lx = threadIdx.x & 7, ly = (threadIdx.x >> 3) & 7, lz = threadIdx.x >> 6;
-  const uint16_t v = gen_voxel(gen, bx * 8 + lx, by * 8 + ly, bz * 8 + lz, n, seed, heights);
-  const unsigned long long b = __ballot(v != 0);
-  __shared__ uint32_t cnt;
-  if (threadIdx.x == 0) cnt = 0;
-  __syncthreads();
-  if ((threadIdx.x & 63u) == 0 && b) atomicAdd(&cnt, (uint32_t)__popcll(b));
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    flags[bid] = cnt ? 1u : 0u;
-    if (cnt) atomicAdd(solid, (unsigned long long)cnt);
+// What the brick kernels need of a generator.  [lo, hi]: the octave sums
+// `sum` for which |fl(fl(sum / norm) - 1/2)| < threshold.  Both roundings are
+// monotone, so these sums form an interval; its ends are found on the host
+// (band_of_sums), and the kernels compare two floats per voxel instead of
+// dividing.
+struct BrickGen {
+  int32_t gen, n;
+  uint32_t seed;
+  int32_t octaves;
+  float base_freq, lo, hi;
+  const int32_t *heights;
+};
+
+__device__ __forceinline__ float lane_value(float v, int lane) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), lane));
+}
+__device__ __forceinline__ float from_lane(float v, uint32_t lane) {
+  return __uint_as_float(
+      (uint32_t)__builtin_amdgcn_ds_bpermute((int)(lane * 4u), (int)__float_as_uint(v)));
+}
+
+// Octave sums of fbm3 over a brick by one wave: lane x + 8 y, sum[z] for the
+// brick's 8 planes, each in fbm3's order of operations.
+// What bounds it is instruction issue: hashing the 8 lattice corners of every
+// voxel (14 hashes per octave, each with two quarter-rate multiplies) took
+// most of the time.  A brick touches at most 3 lattice points per axis when a
+// lattice cell is at least 8 voxels wide (f <= 1/8), so the 27 points of an
+// octave are hashed by 27 lanes at once (two octaves per pass), and each lane
+// fetches its corners by lane permutes.  The x and y interpolation is done
+// once per column, since only the z weight changes along it.  At least 8
+// voxels wide is every octave of scenes of 256 voxels and more; an octave with
+// smaller cells hashes per voxel (value_noise3).
+__device__ __forceinline__ void brick_fbm(const BrickGen &g, uint32_t seed, int32_t x0, int32_t y0,
+                                          int32_t z0, float sum[8]) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const float x = (float)(x0 + (int32_t)(lane & 7u)), y = (float)(y0 + (int32_t)(lane >> 3));
+  // lane o * 8 + z: the z weight and lattice plane (relative to the brick's
+  // first) of octave o at plane z
+  const float fz_l = g.base_freq * (float)(1u << ((lane >> 3) & 3u));
+  const float pz = (float)(z0 + (int32_t)(lane & 7u)) * fz_l;
+  const float flz = __builtin_floorf(pz);
+  const float uz_l = fade(pz - flz);
+  const int32_t dz_l = (int32_t)flz - (int32_t)__builtin_floorf((float)z0 * fz_l);
+  float lattice = 0.0f;
+#pragma unroll
+  for (int z = 0; z < 8; z++) sum[z] = 0.0f;
+  float amp = 1.0f, f = g.base_freq;
+#pragma unroll
+  for (int o = 0; o < 4; o++) {
+    if (o < g.octaves) {
+      const uint32_t so = seed + (uint32_t)o * kOctaveSeedStep;
+      if (f <= 0.125f) {
+        if ((o & 1) == 0) {
+          // lattice points of octaves o (lanes 0..26) and o + 1 (lanes 32..58)
+          const float fl = lane < 32u ? f : f * 2.0f;
+          const uint32_t sl = lane < 32u ? so : so + kOctaveSeedStep;
+          const uint32_t r = lane & 31u, rz = r / 9u, ry = (r - rz * 9u) / 3u,
+                         rx = r - rz * 9u - ry * 3u;
+          const uint32_t ix = (uint32_t)(int32_t)__builtin_floorf((float)x0 * fl) + rx,
+                         iy = (uint32_t)(int32_t)__builtin_floorf((float)y0 * fl) + ry,
+                         iz = (uint32_t)(int32_t)__builtin_floorf((float)z0 * fl) + rz;
+          lattice = hash_unit(nhash32(ix ^ nhash32(iy ^ nhash32(iz ^ sl))));
+        }
+        const float px = x * f, py = y * f;
+        const float flx = __builtin_floorf(px), fly = __builtin_floorf(py);
+        const float ux = fade(px - flx), uy = fade(py - fly);
+        const uint32_t dx = (uint32_t)((int32_t)flx - (int32_t)__builtin_floorf((float)x0 * f)),
+                       dy = (uint32_t)((int32_t)fly - (int32_t)__builtin_floorf((float)y0 * f));
+        const uint32_t at = (uint32_t)(o & 1) * 32u + dx + 3u * dy;
+        auto plane = [&](uint32_t level) {
+          const uint32_t p = at + 9u * level;
+          const float a = lerpf(from_lane(lattice, p), from_lane(lattice, p + 1u), ux);
+          const float b = lerpf(from_lane(lattice, p + 3u), from_lane(lattice, p + 4u), ux);
+          return lerpf(a, b, uy);
+        };
+        const float y0v = plane(0u), y1v = plane(1u);
+        // the last plane of voxels lies in the second cell (uniform)
+        const bool two = __builtin_amdgcn_readlane(dz_l, o * 8 + 7) != 0;
+        const float y2v = two ? plane(2u) : y1v;
+#pragma unroll
+        for (int z = 0; z < 8; z++) {
+          const bool second = __builtin_amdgcn_readlane(dz_l, o * 8 + z) != 0;
+          const float n = lerpf(second ? y1v : y0v, second ? y2v : y1v, lane_value(uz_l, o * 8 + z));
+          const float an = amp * n;
+          sum[z] = sum[z] + an;
+        }
+      } else {
+        for (int z = 0; z < 8; z++) {
+          const float n = value_noise3(x * f, y * f, (float)(z0 + z) * f, so);
+          const float an = amp * n;
+          sum[z] = sum[z] + an;
+        }
+      }
+      amp = amp * 0.5f;
+      f = f * 2.0f;
+    }
   }
 }
 
-__global__ void __launch_bounds__(512) brick_write_kernel(int32_t gen, int32_t n, uint32_t seed,
-                                                          const int32_t *heights, int32_t two_level,
+// The occupancy words of brick (bx, by, bz) by one wave: m[z], bit x + 8 y.
+// False when the brick is empty.
+__device__ __forceinline__ bool brick_words(const BrickGen &g, int32_t bx, int32_t by, int32_t bz,
+                                            uint64_t m[8]) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const int32_t x0 = bx * 8, y0 = by * 8, z0 = bz * 8;
+  int32_t h = 0;
+  if (g.gen != MESO_GEN_CAVES) {
+    // lane x + 8 z: the column's height; the whole brick lies above the
+    // ground when no column reaches its lowest voxels
+    h = g.heights[(int64_t)(z0 + (int32_t)(lane >> 3)) * g.n + x0 + (int32_t)(lane & 7u)];
+    if (__ballot(h > y0) == 0ull) return false;
+  }
+  float sum[8];
+  if (g.gen != MESO_GEN_HEIGHTFIELD)
+    brick_fbm(g, g.gen == MESO_GEN_CAVES ? g.seed : g.seed ^ 0x5bd1e995u, x0, y0, z0, sum);
+  const int32_t y = y0 + (int32_t)(lane >> 3);
+  uint64_t any = 0;
+#pragma unroll
+  for (int z = 0; z < 8; z++) {
+    bool solid;
+    if (g.gen == MESO_GEN_CAVES) {
+      solid = sum[z] >= g.lo && sum[z] <= g.hi;
+    } else {
+      solid = y < __shfl(h, (int)((lane & 7u) + 8u * (uint32_t)z), 64);
+      if (g.gen == MESO_GEN_TERRAIN_CAVES) solid = solid && !(sum[z] >= g.lo && sum[z] <= g.hi);
+    }
+    m[z] = __ballot(solid);
+    any |= m[z];
+  }
+  return any != 0ull;
+}
+
+// Which bricks hold a voxel, and how many voxels are solid: one wave per
+// brick, `per` bricks in turn, so that a workgroup adds to the voxel count
+// once (one add per brick kept the adds to that one word, at a few
+// nanoseconds each, in the way).
+__global__ void __launch_bounds__(256) brick_flags_kernel(BrickGen g, int32_t two_level,
+                                                          uint32_t *flags,
+                                                          unsigned long long *solid,
+                                                          uint64_t n_bricks, uint32_t per) {
+  __shared__ uint32_t wave_solid[4];
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint64_t first = (block_id() * 4u + wave) * per;
+  const int32_t nb = g.n / 8;
+  uint32_t count = 0;
+  for (uint32_t k = 0; k < per && first + k < n_bricks; k++) {
+    int32_t bx, by, bz;
+    brick_of(first + k, nb, two_level != 0, bx, by, bz);
+    uint64_t m[8];
+    const bool any = brick_words(g, bx, by, bz, m);
+    if (any) {
+#pragma unroll
+      for (int z = 0; z < 8; z++) count += (uint32_t)__popcll(m[z]);
+    }
+    if ((threadIdx.x & 63u) == 0) flags[first + k] = any ? 1u : 0u;
+  }
+  if ((threadIdx.x & 63u) == 0) wave_solid[wave] = count;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const uint32_t all = wave_solid[0] + wave_solid[1] + wave_solid[2] + wave_solid[3];
+    if (all) atomicAdd(solid, (unsigned long long)all);
+  }
+}
+
+// Writes the slots, and the masks and voxels of the bricks that hold a voxel:
+// one wave per brick, `per` bricks in turn.  The words are computed again (a
+// third of the bricks at most need it) rather than kept, which would take 64
+// bytes per brick cell.  A voxel's material depends on its height alone, so a
+// lane writes one row of 8 voxels (y, z) from its byte of the words: one
+// 1 KiB store per brick.
+__global__ void __launch_bounds__(256) brick_write_kernel(BrickGen g, int32_t two_level,
                                                           const uint32_t *flags,
                                                           const uint32_t *prefix,
                                                           const uint32_t *node_ids,
                                                           uint32_t *slots, uint64_t *masks,
-                                                          uint16_t *voxels, uint64_t n_bricks) {
-  const int32_t nb = n / 8;
-  const uint64_t ordered = block_id();
-  if (ordered >= n_bricks) return;  // uniform over the workgroup
-  if (two_level) {
-    // bricks of empty nodes have no slot table
-    const uint32_t node = node_ids[ordered / 4096u];
-    if (node == kEmptySlot) return;
-    if (threadIdx.x == 0)
-      slots[(uint64_t)node * 4096u + ordered % 4096u] = flags[ordered] ? prefix[ordered] : kEmptySlot;
-  } else if (threadIdx.x == 0) {
-    slots[ordered] = flags[ordered] ? prefix[ordered] : kEmptySlot;
+                                                          uint16_t *voxels, uint64_t n_bricks,
+                                                          uint32_t per) {
+  const int32_t nb = g.n / 8;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint64_t first = (block_id() * 4u + wave) * per;
+  for (uint32_t k = 0; k < per && first + k < n_bricks; k++) {
+    const uint64_t ordered = first + k;
+    const bool live = flags[ordered] != 0u;
+    uint64_t cell = ordered;
+    if (two_level) {
+      // bricks of empty nodes have no slot table
+      const uint32_t node = node_ids[ordered / 4096u];
+      if (node == kEmptySlot) continue;
+      cell = (uint64_t)node * 4096u + ordered % 4096u;
+    }
+    if (lane == 0) slots[cell] = live ? prefix[ordered] : kEmptySlot;
+    if (!live) continue;
+    int32_t bx, by, bz;
+    brick_of(ordered, nb, two_level != 0, bx, by, bz);
+    uint64_t m[8];
+    brick_words(g, bx, by, bz, m);
+    uint64_t w = m[0];
+#pragma unroll
+    for (uint32_t z = 1; z < 8u; z++) w = (lane >> 3) == z ? m[z] : w;
+    const uint64_t slot = prefix[ordered];
+    if ((lane & 7u) == 0) masks[slot * 8u + (lane >> 3)] = w;
+    const uint32_t row = (uint32_t)(w >> (8u * (lane & 7u))) & 0xFFu;
+    const int32_t y = by * 8 + (int32_t)(lane & 7u);
+    const uint32_t mat = g.gen == MESO_GEN_CAVES ? caves_material(y) : height_band(y, g.n);
+    uint32_t v[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      v[j] = (((row >> (2 * j)) & 1u) | (((row >> (2 * j + 1)) & 1u) << 16)) * mat;
+    *(uint4 *)(voxels + slot * 512u + 8u * lane) = make_uint4(v[0], v[1], v[2], v[3]);
   }
-  if (!flags[ordered]) return;
-  int32_t bx, by, bz;
-  brick_of(ordered, nb, two_level != 0, bx, by, bz);
-  const int32_t lx = threadIdx.x & 7, ly = (threadIdx.x >> 3) & 7, lz = threadIdx.x >> 6;
-  const uint16_t v = gen_voxel(gen, bx * 8 + lx, by * 8 + ly, bz * 8 + lz, n, seed, heights);
-  const unsigned long long b = __ballot(v != 0);
-  const uint64_t slot = prefix[ordered];
-  voxels[slot * 512u + threadIdx.x] = v;
-  if ((threadIdx.x & 63u) == 0) masks[slot * 8u + lz] = (uint64_t)b;
 }
 
 __global__ void node_flags_kernel(const uint32_t *brick_flags, uint32_t *node_flags) {
@@ -448,6 +592,106 @@ __global__ void __launch_bounds__(512) edit_chunks_kernel(DevScene s, int32_t ki
 
 using namespace meso;
 
+// the sums whose noise value lies within `thr` of 1/2 (see BrickGen): the
+// first and last positive float of the interval, found by bisection of the
+// float's bits on both sides of the middle
+static bool in_band(float sum, float norm, float thr) {
+  float c = sum / norm;
+  c = c - 0.5f;
+  return std::fabs(c) < thr;
+}
+static float band_end(float norm, float thr, uint32_t outside) {
+  float mid = 0.5f * norm;
+  uint32_t in, out = outside;
+  std::memcpy(&in, &mid, 4);
+  while (in > out ? in - out > 1u : out - in > 1u) {
+    const uint32_t probe = in > out ? out + (in - out) / 2u : in + (out - in) / 2u;
+    float v;
+    std::memcpy(&v, &probe, 4);
+    if (in_band(v, norm, thr)) in = probe;
+    else out = probe;
+  }
+  float r;
+  std::memcpy(&r, &in, 4);
+  return r;
+}
+
+// Fills sc's slots, masks and voxels (and top table) from the generator.
+// scratch: the words meso_scene_generate counts out, first the totals.
+static meso_status generate_bricks(meso_scene *sc, int32_t gen, uint32_t seed, uint32_t *scratch,
+                                   hipStream_t stream) {
+  const int32_t n = sc->n, nb = n / 8, nt = n / 128;
+  const bool two = sc->kind == MESO_SCENE_TWO_LEVEL_U16;
+  const uint64_t cells = (uint64_t)nb * nb * nb, n_top = two ? (uint64_t)nt * nt * nt : 0;
+  uint32_t *totals = scratch;  // [0] bricks, [1] nodes, [2..3] solid voxels
+  uint32_t *flags = totals + 4, *prefix = flags + cells;
+  uint32_t *node_flags = prefix + cells, *node_prefix = node_flags + n_top;
+  int32_t *heights = (int32_t *)(node_prefix + n_top);
+  uint32_t *ws = (uint32_t *)heights + (gen != MESO_GEN_CAVES ? (uint64_t)n * n : 0);
+  meso_status st = launch_zero(totals, 16, stream);
+  if (st != MESO_OK) return st;
+  if (gen != MESO_GEN_CAVES) {
+    hipLaunchKernelGGL(heights_kernel, dim3((uint32_t)(((uint64_t)n * n + 255) / 256)), dim3(256),
+                       0, stream, heights, n, seed, gen);
+    MESO_HIP(hipGetLastError());
+  }
+  BrickGen g{};
+  g.gen = gen;
+  g.n = n;
+  g.seed = seed;
+  g.heights = heights;
+  g.octaves = gen == MESO_GEN_CAVES ? 4 : 3;
+  g.base_freq = gen == MESO_GEN_CAVES ? 1.0f / 64.0f : 8.0f / (float)n;
+  const float norm = gen == MESO_GEN_CAVES ? 1.875f : 1.75f;  // 1 + 1/2 + 1/4 (+ 1/8)
+  const float thr = gen == MESO_GEN_CAVES ? kCavesBand : kTunnelBand;
+  g.lo = band_end(norm, thr, 0u);
+  g.hi = band_end(norm, thr, 0x40000000u);
+  // a wave takes several bricks once there are more than 16 waves per CU
+  const uint32_t waves = (uint32_t)sc->ctx->props.multiProcessorCount * 16u;
+  uint32_t per = (uint32_t)(cells / waves);
+  per = per < 1u ? 1u : (per > 16u ? 16u : per);
+  const dim3 grid = grid_1d((cells + 4u * per - 1) / (4u * per));
+  hipLaunchKernelGGL(brick_flags_kernel, grid, dim3(256), 0, stream, g, two ? 1 : 0, flags,
+                     (unsigned long long *)(totals + 2), cells, per);
+  MESO_HIP(hipGetLastError());
+  st = scan_u32(flags, prefix, cells, totals, ws, stream);
+  if (st != MESO_OK) return st;
+  if (two) {
+    hipLaunchKernelGGL(node_flags_kernel, dim3((uint32_t)n_top), dim3(256), 0, stream, flags,
+                       node_flags);
+    MESO_HIP(hipGetLastError());
+    st = scan_u32(node_flags, node_prefix, n_top, totals + 1, ws, stream);
+    if (st != MESO_OK) return st;
+  }
+  uint32_t t[4];
+  MESO_HIP(hipMemcpyAsync(t, totals, sizeof(t), hipMemcpyDeviceToHost, stream));
+  MESO_HIP(hipStreamSynchronize(stream));
+  const uint64_t n_bricks = t[0], n_nodes = t[1];
+  sc->n_bricks = (int64_t)n_bricks;
+  sc->n_nodes = (int64_t)n_nodes;
+  sc->solid = (int64_t)((uint64_t)t[2] | ((uint64_t)t[3] << 32));
+  MESO_CHECK(n_bricks < (1ull << 29), MESO_ERR_OUT_OF_MEMORY, "%llu bricks exceed 2^29",
+             (unsigned long long)n_bricks);
+  if (two) {
+    MESO_HIP(hipMalloc((void **)&sc->top, n_top * 4));
+    hipLaunchKernelGGL(node_ids_kernel, dim3((uint32_t)((n_top + 255) / 256)), dim3(256), 0,
+                       stream, node_flags, node_prefix, sc->top, n_top);
+    MESO_HIP(hipGetLastError());
+    MESO_HIP(hipMalloc((void **)&sc->slots, std::max<uint64_t>(n_nodes, 1) * 4096 * 4));
+    sc->bytes += n_top * 4 + n_nodes * 4096 * 4;
+  } else {
+    MESO_HIP(hipMalloc((void **)&sc->slots, cells * 4));
+    sc->bytes += cells * 4;
+  }
+  MESO_HIP(hipMalloc((void **)&sc->masks, std::max<uint64_t>(n_bricks, 1) * 64));
+  MESO_HIP(hipMalloc((void **)&sc->voxels, std::max<uint64_t>(n_bricks, 1) * 1024));
+  sc->bytes += n_bricks * (64 + 1024);
+  hipLaunchKernelGGL(brick_write_kernel, grid, dim3(256), 0, stream, g, two ? 1 : 0, flags, prefix,
+                     sc->top, sc->slots, sc->masks, sc->voxels, cells, per);
+  MESO_HIP(hipGetLastError());
+  return MESO_OK;
+}
+
 static meso_status gen_free(meso_scene *sc, meso_status st) {
   if (sc) {
     hipSetDevice(sc->ctx->device);
@@ -538,66 +782,19 @@ meso_status meso_scene_generate(meso_context *ctx, const meso_generate_desc *d, 
   sc->ctx = ctx;
   sc->kind = two ? MESO_SCENE_TWO_LEVEL_U16 : MESO_SCENE_BRICKMAP_U16;
   sc->n = n;
-  int32_t *heights = nullptr;
-  uint32_t *flags = nullptr, *prefix = nullptr, *node_flags = nullptr, *node_prefix = nullptr;
-  unsigned long long *solid = nullptr;
-  if (d->generator != MESO_GEN_CAVES) {
-    GEN_HIP(hipMallocAsync((void **)&heights, (uint64_t)n * n * 4, stream));
-    hipLaunchKernelGGL(heights_kernel, dim3((uint32_t)(((uint64_t)n * n + 255) / 256)), dim3(256),
-                       0, stream, heights, n, seed, d->generator);
-    GEN_HIP(hipGetLastError());
-  }
-  GEN_HIP(hipMallocAsync((void **)&flags, n_brick_cells * 4, stream));
-  GEN_HIP(hipMallocAsync((void **)&prefix, n_brick_cells * 4, stream));
-  GEN_HIP(hipMallocAsync((void **)&solid, 8, stream));
-  GEN_TRY(launch_zero(solid, 8, stream));
-  hipLaunchKernelGGL(brick_flags_kernel, grid_1d(n_brick_cells), dim3(512), 0, stream,
-                     d->generator, n, seed, heights, two ? 1 : 0, flags, solid, n_brick_cells);
-  GEN_HIP(hipGetLastError());
-  uint64_t n_bricks = 0;
-  GEN_TRY(scan_u32(flags, prefix, n_brick_cells, &n_bricks, stream));
-  uint64_t n_nodes = 0;
   const int32_t nt = n / 128;
   const uint64_t n_top = two ? (uint64_t)nt * nt * nt : 0;
-  if (two) {
-    GEN_HIP(hipMallocAsync((void **)&node_flags, n_top * 4, stream));
-    GEN_HIP(hipMallocAsync((void **)&node_prefix, n_top * 4, stream));
-    hipLaunchKernelGGL(node_flags_kernel, dim3((uint32_t)n_top), dim3(256), 0, stream, flags,
-                       node_flags);
-    GEN_HIP(hipGetLastError());
-    GEN_TRY(scan_u32(node_flags, node_prefix, n_top, &n_nodes, stream));
-    GEN_HIP(hipMalloc((void **)&sc->top, n_top * 4));
-    hipLaunchKernelGGL(node_ids_kernel, dim3((uint32_t)((n_top + 255) / 256)), dim3(256), 0,
-                       stream, node_flags, node_prefix, sc->top, n_top);
-    GEN_HIP(hipGetLastError());
-    GEN_HIP(hipMalloc((void **)&sc->slots, std::max<uint64_t>(n_nodes, 1) * 4096 * 4));
-    sc->bytes += n_top * 4 + n_nodes * 4096 * 4;
-  } else {
-    GEN_HIP(hipMalloc((void **)&sc->slots, n_brick_cells * 4));
-    sc->bytes += n_brick_cells * 4;
-  }
-  GEN_HIP(hipMalloc((void **)&sc->masks, std::max<uint64_t>(n_bricks, 1) * 64));
-  GEN_HIP(hipMalloc((void **)&sc->voxels, std::max<uint64_t>(n_bricks, 1) * 1024));
-  sc->bytes += n_bricks * (64 + 1024);
-  hipLaunchKernelGGL(brick_write_kernel, grid_1d(n_brick_cells), dim3(512), 0, stream,
-                     d->generator, n, seed, heights, two ? 1 : 0, flags, prefix, sc->top, sc->slots,
-                     sc->masks, sc->voxels, n_brick_cells);
-  GEN_HIP(hipGetLastError());
-  unsigned long long s = 0;
-  GEN_HIP(hipMemcpyAsync(&s, solid, 8, hipMemcpyDeviceToHost, stream));
-  GEN_HIP(hipStreamSynchronize(stream));
-  if (heights) hipFreeAsync(heights, stream);
-  hipFreeAsync(flags, stream);
-  hipFreeAsync(prefix, stream);
-  hipFreeAsync(solid, stream);
-  if (node_flags) hipFreeAsync(node_flags, stream);
-  if (node_prefix) hipFreeAsync(node_prefix, stream);
-  GEN_HIP(hipStreamSynchronize(stream));
-  sc->n_bricks = (int64_t)n_bricks;
-  sc->n_nodes = (int64_t)n_nodes;
-  sc->solid = (int64_t)s;
-  MESO_CHECK(n_bricks < (1ull << 29), MESO_ERR_OUT_OF_MEMORY, "%llu bricks exceed 2^29",
-             (unsigned long long)n_bricks);
+  // one scratch allocation: totals (bricks, nodes, solid voxels), flags and
+  // prefix per brick cell and per node, column heights, the scans' sums
+  const uint64_t words = 4 + 2 * n_brick_cells + 2 * n_top +
+                         (d->generator != MESO_GEN_CAVES ? (uint64_t)n * n : 0) +
+                         scan_ws_words(n_brick_cells);
+  uint32_t *scratch = nullptr;
+  GEN_HIP(hipMallocAsync((void **)&scratch, words * 4, stream));
+  const meso_status st = generate_bricks(sc, d->generator, seed, scratch, stream);
+  // the stream is idle on success; after a failure gen_free waits for it
+  (void)hipFreeAsync(scratch, stream);
+  if (st != MESO_OK) return gen_free(sc, st);
   GEN_TRY(build_coarse(sc, stream));
   *out = sc;
   return MESO_OK;
