@@ -140,6 +140,7 @@ struct meso_scene {
   uint32_t *occ128 = nullptr;
   uint64_t *groups = nullptr;
   uint64_t *bricks32 = nullptr;  // see DevScene::bricks32
+  void *derived = nullptr;       // holds blocks, slot_cell and the levels above
   int64_t n_bricks = 0;
   int64_t n_nodes = 0;
   uint64_t bytes = 0;
