@@ -515,14 +515,16 @@ meso_status meso_chunk_pool_arrays(meso_chunk_pool *pool, meso_pool_arrays *out)
 typedef struct meso_raster meso_raster;
 typedef struct meso_raster_stats {
   uint32_t size;           /* sizeof(meso_raster_stats) */
-  uint32_t small_quads;    /* last frame: quads of at most 64 pixels, tested by one lane */
-  uint32_t large_quads;    /* last frame: larger quads, tested by a wave (up to 4096 pixels)
-                              or cut into segments of 16384 pixels */
-  uint32_t segments;       /* last frame: the segments */
-  uint32_t overflow_quads; /* last frame: quads tested by one lane (segment list full) */
+  /* quads of the last frame that were neither turned away nor outside the frame nor hidden
+     behind what was drawn before them, by the pixels of their bounds with a margin of one: */
+  uint32_t small_quads;    /* at most 64 pixels */
+  uint32_t large_quads;    /* more */
+  uint32_t segments;       /* quads listed, so that the tests of all their pixels are
+                              shared out evenly over the device */
+  uint32_t overflow_quads; /* quads tested where they were found (the list was full) */
 } meso_raster_stats;
-/* Scratch for frames up to max_width x max_height (8 B per pixel plus a
- * 64 MiB segment list). */
+/* Scratch for frames up to max_width x max_height (about 20 B per pixel plus
+ * 144 MiB of lists). */
 meso_status meso_raster_create(meso_context *ctx, int32_t max_width, int32_t max_height,
                                meso_raster **out);
 meso_status meso_raster_destroy(meso_raster *raster);
