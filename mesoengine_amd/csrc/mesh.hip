@@ -1,6 +1,6 @@
 // Culled-face and greedy meshing of 32^3 chunks on gfx950.
 //
-// One workgroup (256 lanes) meshes one chunk:
+// One workgroup (256 to 1024 lanes) meshes one chunk:
 //  1. Row masks.  Each lane loads 8 voxels of a 32-voxel row with one vector
 //     load, plus the same 8 voxels of the +y row and of the +z row, and forms
 //     8-bit masks in registers: occupancy and material equality with the +x,
@@ -20,9 +20,8 @@
 //     the canonical greedy merge (scan row-major, width first, then height):
 //     a quad's height never depends on cells claimed by other quads, because
 //     quads created before it never share its columns below its first row.
-//     Counting is popcounts of the new-run starts; emitting keeps one packed
-//     record (first row, canonical index) per open quad and writes each quad
-//     when its segment stops.
+//     Every row's new cells and ending quads stay in LDS; the emission then
+//     takes a lane per quad, over the whole workgroup.
 //  3. Batched mode: chunks come from an atomic ticket, and each chunk finds
 //     its output offset by an ordered decoupled look-back over the chunks
 //     ticketed before it, so one persistent launch writes one compact quad
@@ -35,7 +34,17 @@
 namespace meso {
 
 constexpr int kPlanes = 192;  // 6 faces x 32 slices
-constexpr int kMeshBlock = 256;
+// Threads per workgroup.  A single chunk and a pool's loads (about a chunk per
+// CU) are bound by one chunk's latency, so they take the whole CU: one greedy
+// chunk of 11,839 quads 61.5 -> 31.3 us, the pool's 256 loads 45.9 -> 24.8 us
+// (with 256 threads and one emitting lane per plane before).  Batches are
+// bound by issue: 4096 greedy chunks 265 -> 254 us at 512 threads, two
+// workgroups per CU by LDS (at 1024, one per CU by registers, 331 us; two by
+// a bound of 64 registers 256 us).  A culled batch keeps five workgroups.
+constexpr int kMeshBlock = 256;     // culled batches
+constexpr int kGreedyBlock = 512;   // greedy batches
+constexpr int kChunkBlock = 1024;   // single chunks and pool loads
+
 
 struct ChunkAddr {
   const void *base;
@@ -196,20 +205,33 @@ enum : int {
   kEy = 64 * kZY,
   kEz = 96 * kZY,
   kOT = 128 * kZY,
-  kEyT = kOT + 1024,
-  kEzT = kOT + 2048,
-  kMaskWords = kOT + 3072
+  kEyT = 160 * kZY,
+  kEzT = 192 * kZY,
+  kMaskWords = 224 * kZY
 };
 
 struct MeshLds {
   uint32_t M[kMaskWords];
-  uint32_t pex[kPlanes];  // culled: exclusive quad offset of each plane in the chunk
-  uint32_t occ[kPlanes];  // culled: bit v set when row v of the plane has a face
-  uint32_t scan[kMeshBlock / 64];
+  uint32_t pex[kPlanes];  // exclusive quad offset of each plane in the chunk
+  uint32_t occ[kPlanes];  // culled: bit v set when row v of the plane has a face;
+                          // greedy: bit v set when quads end in row v
+  uint32_t scan[16];
   uint32_t bslot[64];  // scene chunks: slots of the chunk's 4x4x4 bricks
   uint32_t chunk;
   uint32_t base_lo, base_hi;
 };
+
+// Greedy meshing: what the row sweep of each plane leaves for the emission.
+// Neighbouring lanes of the emission read neighbouring rows of one plane, so
+// rows lie an odd number of words apart (at 192, a multiple of the 32 banks,
+// all rows of a plane shared one bank).
+constexpr int kRowWords = kPlanes + 1;
+struct GreedyLds : MeshLds {
+  uint32_t avail[32 * kRowWords];  // [v][plane]: cells of row v that start quads there
+  uint32_t ends[32 * kRowWords];   // [v][plane]: starts of the quads whose last row is v
+};
+template <bool GREEDY>
+using LdsOf = typename std::conditional<GREEDY, GreedyLds, MeshLds>::type;
 
 // 32x32 bit transpose across the 32 lanes of a half wave: lane y holds row y
 // (bit x = element [y][x]) and gets back column y (bit x = element [x][y]).
@@ -240,10 +262,10 @@ __device__ __forceinline__ uint32_t row_or(uint32_t piece) {
 }
 
 // Step 1: masks.  Wave w handles blocks of 16 rows (rows r = y + 32 z).
-template <int ES, class Rows>
+template <int ES, int T, class Rows>
 __device__ __forceinline__ void build_masks(MeshLds &L, const Rows &a) {
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  constexpr uint32_t nwaves = kMeshBlock / 64;
+  constexpr uint32_t nwaves = T / 64;
   const int k = (int)(lane & 3u);
   // two row blocks per trip: all their loads are issued before either
   // block's arithmetic, so a trip waits on memory once
@@ -310,7 +332,7 @@ __device__ __forceinline__ void build_masks(MeshLds &L, const Rows &a) {
     constexpr int dst[3] = {kOT, kEyT, kEzT};
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-      L.M[dst[k] + z * 32u + y] = transpose32(rows[k], y);
+      L.M[dst[k] + z * kZY + y] = transpose32(rows[k], y);
     }
   }
   __syncthreads();
@@ -319,7 +341,7 @@ __device__ __forceinline__ void build_masks(MeshLds &L, const Rows &a) {
 // Masks of scene chunk (ox, oy, oz) / 32: the slots of its 64 bricks are
 // resolved first, one lane each, so that the row loads do not wait on the
 // brick lookups.
-template <int ES, int KIND>
+template <int ES, int T, int KIND>
 __device__ __forceinline__ void build_masks(MeshLds &L, const SceneRows<KIND> &a) {
   const uint32_t t = threadIdx.x;
   if (t < 64u)
@@ -327,7 +349,7 @@ __device__ __forceinline__ void build_masks(MeshLds &L, const SceneRows<KIND> &a
                                   (a.oy >> 3) + (int32_t)((t >> 2) & 3u),
                                   (a.oz >> 3) + (int32_t)(t >> 4));
   __syncthreads();
-  build_masks<ES>(L, SlotRows{L.bslot, a.s.voxels});
+  build_masks<ES, T>(L, SlotRows{L.bslot, a.s.voxels});
 }
 
 // Offsets of plane (f, s) in the mask planes.  z faces: (u,v) = (x,y) and
@@ -357,7 +379,7 @@ __device__ __forceinline__ PlaneView plane_view(int f, int s) {
     p.nb = inside ? kOT + ns : -1;
     p.eu = kEyT + s;
     p.ev = kEzT + s;
-    p.stride = 32;
+    p.stride = kZY;
   }
   return p;
 }
@@ -410,161 +432,52 @@ __device__ __forceinline__ uint32_t segment_fill(uint32_t marks, uint32_t cont) 
   return up | dn;
 }
 
-// Step 2a: quad count of plane t; culled meshing also returns the plane's
-// non-empty rows in `occ`.
-template <bool GREEDY>
+// Step 2a, culled: quad count of plane t; its non-empty rows in `occ`.
 __device__ __forceinline__ uint32_t plane_count(const MeshLds &L, int t, uint32_t &occ) {
   const PlaneView p = plane_view(t >> 5, t & 31);
   uint32_t count = 0;
   occ = 0;
-  if (!GREEDY) {
 #pragma unroll 8
-    for (int v = 0; v < 32; v++) {
-      const uint32_t c = (uint32_t)__popc(face_row(L, p, v));
-      count += c;
-      occ |= (c != 0u ? 1u : 0u) << v;
-    }
-    return count;
-  }
-  uint32_t open = 0, starts = 0, ev_prev = 0;
-#pragma unroll 4
   for (int v = 0; v < 32; v++) {
-    const uint32_t F = face_row_at(L, p, v * p.stride);
-    const uint32_t eh = L.M[p.eu + v * p.stride];
-    if (v > 0) {
-      const uint32_t dead = segment_fill(open & ~(F & ev_prev), open & ~starts) & open;
-      open &= ~dead;
-      starts &= ~dead;
-    }
-    const uint32_t avail = F & ~open;
-    const uint32_t st = avail & ~((avail & eh) << 1);
-    count += (uint32_t)__popc(st);
-    open |= avail;
-    starts |= st;
-    ev_prev = L.M[p.ev + v * p.stride];
+    const uint32_t c = (uint32_t)__popc(face_row(L, p, v));
+    count += c;
+    occ |= (c != 0u ? 1u : 0u) << v;
   }
   return count;
 }
 
-// Start rows of the open quads, bit-sliced: bit u of row[k] is bit k of the
-// first row of the quad that starts at u (kept in registers, no table).
-struct StartRows {
-  uint32_t row[5];
-};
-
-__device__ __forceinline__ void record_starts(StartRows &r, uint32_t st, int v) {
-#pragma unroll
-  for (int k = 0; k < 5; k++) r.row[k] = (r.row[k] & ~st) | (((v >> k) & 1) ? st : 0u);
-}
-
-__device__ __forceinline__ uint32_t start_row(const StartRows &r, uint32_t u) {
-  uint32_t v = __builtin_amdgcn_ubfe(r.row[0], u, 1u);
-#pragma unroll
-  for (int k = 1; k < 5; k++) v |= __builtin_amdgcn_ubfe(r.row[k], u, 1u) << k;
-  return v;
-}
-
-// pack_quad with plane (f, s)'s axes resolved once:
-// quad = fixed | u << su | v << sv | (w - 1) << 15 | (h - 1) << 20.
-struct PlanePack {
-  uint32_t fixed, su, sv;
-};
-
-__device__ __forceinline__ PlanePack plane_pack(int f, int s) {
-  PlanePack p;
-  if (f < 2) {  // (x, y, z) = (u, v, s)
-    p.su = 0;
-    p.sv = 5;
-    p.fixed = (uint32_t)s << 10;
-  } else if (f < 4) {  // (u, s, v)
-    p.su = 0;
-    p.sv = 10;
-    p.fixed = (uint32_t)s << 5;
-  } else {  // (s, u, v)
-    p.su = 5;
-    p.sv = 10;
-    p.fixed = (uint32_t)s;
-  }
-  p.fixed |= (uint32_t)f << 25;
-  return p;
-}
-
-// The quad of the segment that starts at u (its columns: u and the `cont`
-// bits above it), first row v, last row vend - 1.  (cont >> u) >> 1 is 0 at
-// u = 31, where the width is 1.
-__device__ __forceinline__ uint32_t closed_quad(const PlanePack &pk, uint32_t cont, uint32_t u,
-                                                uint32_t v, uint32_t vend) {
-  const uint32_t wm1 = (uint32_t)__builtin_ctz(~((cont >> u) >> 1));
-  return pk.fixed | (u << pk.su) | (v << pk.sv) | (wm1 << 15) | ((vend - v - 1u) << 20);
-}
-
-// Close the quads whose start bits are in `bits` (their last row is
-// vend - 1), in ascending u, at out[base + count ...]; CHECK: stop writing at
-// cap (a caller that knows the plane fits passes false and skips the tests).
-template <bool CHECK>
-__device__ __forceinline__ void close_quads(const StartRows &r, const PlanePack &pk, uint32_t bits,
-                                            uint32_t open, uint32_t starts, uint32_t vend,
-                                            uint32_t *out, uint64_t base, uint64_t cap,
-                                            uint32_t &count) {
-  const uint32_t cont = open & ~starts;
-  while (bits) {  // two quads per trip
-    const uint32_t u1 = (uint32_t)__builtin_ctz(bits);
-    bits &= bits - 1;
-    const bool two = bits != 0u;
-    const uint32_t u2 = two ? (uint32_t)__builtin_ctz(bits) : u1;
-    bits &= two ? bits - 1 : bits;
-    const uint32_t q1 = closed_quad(pk, cont, u1, start_row(r, u1), vend);
-    const uint32_t q2 = closed_quad(pk, cont, u2, start_row(r, u2), vend);
-    const uint64_t k = base + count;
-    count += two ? 2u : 1u;
-    if (!CHECK || k < cap) out[k] = q1;
-    if (two && (!CHECK || k + 1 < cap)) out[k + 1] = q2;
-  }
-}
-
-// Step 2b, greedy: write the quads of plane t at out[base ...] in canonical
-// order: by the row where they end, then by start u (the order the sweep
-// closes them in).
-template <bool CHECK>
-__device__ __forceinline__ void plane_emit_greedy(MeshLds &L, int t, uint32_t *out, uint64_t base,
-                                                  uint64_t cap) {
-  const int f = t >> 5, s = t & 31;
-  const PlaneView p = plane_view(f, s);
-  const PlanePack pk = plane_pack(f, s);
+// Step 2a, greedy: the row sweep of plane t.  Returns its quad count and, in
+// `occ`, the rows in which quads end; leaves every row's new cells and ending
+// quads in L for the emission.
+__device__ __forceinline__ uint32_t plane_sweep(GreedyLds &L, int t, uint32_t &occ) {
+  const PlaneView p = plane_view(t >> 5, t & 31);
   uint32_t count = 0;
+  occ = 0;
   uint32_t open = 0, starts = 0, ev_prev = 0;
-  StartRows r = {{0u, 0u, 0u, 0u, 0u}};
   int off = 0;  // v * stride, kept as a running sum (no multiply per row)
+#pragma unroll 4
   for (int v = 0; v < 32; v++, off += p.stride) {
     const uint32_t F = face_row_at(L, p, off);
     const uint32_t eh = L.M[p.eu + off];
-    const uint32_t ev = L.M[p.ev + off];
     if (v > 0) {
       const uint32_t dead = segment_fill(open & ~(F & ev_prev), open & ~starts) & open;
-      close_quads<CHECK>(r, pk, starts & dead, open, starts, (uint32_t)v, out, base, cap, count);
+      const uint32_t ends = starts & dead;
+      L.ends[(v - 1) * kRowWords + t] = ends;
+      occ |= (ends != 0u ? 1u : 0u) << (v - 1);
       open &= ~dead;
       starts &= ~dead;
     }
     const uint32_t avail = F & ~open;
+    L.avail[v * kRowWords + t] = avail;
     const uint32_t st = avail & ~((avail & eh) << 1);
+    count += (uint32_t)__popc(st);
     open |= avail;
     starts |= st;
-    record_starts(r, st, v);
-    ev_prev = ev;
+    ev_prev = L.M[p.ev + off];
   }
-  close_quads<CHECK>(r, pk, starts, open, starts, 32u, out, base, cap, count);
-}
-
-// Step 2b, greedy: the quads of plane t (`total` of them, from plane_count)
-// at out[base ...], written unchecked when they all fit below cap.  (Culled
-// meshing shares its faces out over the whole workgroup instead:
-// culled_emit_balanced.)
-__device__ __forceinline__ void plane_emit(MeshLds &L, int t, uint32_t *out, uint64_t base,
-                                           uint64_t cap, uint32_t total) {
-  if (base + total <= cap)
-    plane_emit_greedy<false>(L, t, out, base, cap);
-  else
-    plane_emit_greedy<true>(L, t, out, base, cap);
+  L.ends[31 * kRowWords + t] = starts;
+  occ |= (starts != 0u ? 1u : 0u) << 31;
+  return count;
 }
 
 // position of the r-th (0-based) set bit of x; x has more than r set bits
@@ -580,6 +493,12 @@ __device__ __forceinline__ int select_bit(uint32_t x, uint32_t r) {
     }
   }
   return pos;
+}
+
+// the same for small r: one bit dropped per trip
+__device__ __forceinline__ uint32_t nth_bit(uint32_t x, uint32_t r) {
+  for (; r; r--) x &= x - 1u;
+  return (uint32_t)__builtin_ctz(x);
 }
 
 // the last plane whose quad offset is <= q (offsets ascend and repeat over
@@ -604,9 +523,10 @@ __device__ __forceinline__ int plane_of(const MeshLds &L, uint32_t q) {
 // non-empty rows (occ); it crosses to the next plane by the same search.
 constexpr uint32_t kRun = 8;
 
+template <int T>
 __device__ __forceinline__ void culled_emit_balanced(const MeshLds &L, uint32_t total,
                                                      uint32_t *out, uint64_t base, uint64_t cap) {
-  for (uint32_t q0 = threadIdx.x * kRun; q0 < total; q0 += kMeshBlock * kRun) {
+  for (uint32_t q0 = threadIdx.x * kRun; q0 < total; q0 += (uint32_t)T * kRun) {
     const uint32_t q1 = q0 + kRun < total ? q0 + kRun : total;
     int pl = plane_of(L, q0);
     PlaneView p = plane_view(pl >> 5, pl & 31);
@@ -644,7 +564,86 @@ __device__ __forceinline__ void culled_emit_balanced(const MeshLds &L, uint32_t 
   }
 }
 
+// Step 2b, greedy: the chunk's quads at out[base ...] in canonical order, a
+// lane per quad.  The order is by plane, then by the row v where the quad
+// ends, then by start u, so the quads of one (plane, row) are consecutive.
+// The planes' lanes mark the place of every (plane, row) that ends quads, in
+// windows of kMarks places (over the mask planes that only the sweep needed);
+// a lane's (plane, row) is the last mark at or before its place.  A row ends
+// at most 32 quads, so that mark lies in the lane's group of 64 or the group
+// before.  The quad's first row is the last row up to v in which a quad starts
+// at u, and its width the run of new cells joined there.
+// Issue bounds it, some 245 instructions per 64 quads; one lane per plane,
+// writing each quad as its sweep closed it, left a wave waiting for its busiest
+// plane in every row.  Also measured: four rows read per search step 3% longer;
+// a list of (plane, v, u) written by the planes' lanes instead of marks 6 times
+// longer on a chunk of 11,839 quads, whose planes differ that much.
+constexpr uint32_t kMarks = 4096u, kMarkStep = kMarks - 64u;
+static_assert(kEy + kMarks / 2u <= kEyT, "the marks lie over Ey, Ez and OT");
+
+template <int T>
+__device__ __forceinline__ void greedy_emit(GreedyLds &L, uint32_t total, uint32_t *out,
+                                            uint64_t base, uint64_t cap) {
+  const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+  uint16_t *marks = (uint16_t *)(L.M + kEy);  // marks[64 + q - w0]
+  uint32_t *marks2 = L.M + kEy;
+  for (uint32_t w0 = 0; w0 < total; w0 += kMarkStep) {  // uniform
+    for (uint32_t k = t; k < kMarks / 2u; k += (uint32_t)T) marks2[k] = 0u;
+    __syncthreads();
+    if (t < (uint32_t)kPlanes) {
+      uint32_t at = L.pex[t] + 64u - w0;  // wraps below the window
+      for (uint32_t rows = L.occ[t]; rows; rows &= rows - 1u) {
+        const uint32_t v = (uint32_t)__builtin_ctz(rows);
+        if (at < kMarks) marks[at] = (uint16_t)(((v << 8) | t) + 1u);
+        at += (uint32_t)__popc(L.ends[v * kRowWords + t]);
+      }
+    }
+    __syncthreads();
+    const uint32_t len = total - w0 < kMarkStep ? total - w0 : kMarkStep;
+    for (uint32_t g = wave * 64u; g < len; g += (uint32_t)T) {
+      const uint32_t mark = marks[64u + g + lane], prev = marks[g + lane];
+      const uint64_t upto = __ballot(mark != 0u) & (~0ull >> (63u - lane));
+      const uint64_t before = __ballot(prev != 0u);
+      const uint32_t p1 = upto ? 63u - (uint32_t)__builtin_clzll(upto) : 0u;
+      const uint32_t p0 = before ? 63u - (uint32_t)__builtin_clzll(before) : 0u;
+      const uint32_t m1 = (uint32_t)__shfl((int)mark, (int)p1, 64),
+                     m0 = (uint32_t)__builtin_amdgcn_readlane((int)prev, (int)p0);
+      const uint32_t own = (upto ? m1 : m0) - 1u;
+      const uint32_t r = upto ? lane - p1 : lane + 64u - p0;  // the quad's place in its row
+      const uint64_t k = base + w0 + g + lane;
+      if (g + lane < len && k < cap) {
+        // the plane's axes by selects (a branch per axis ran all three sides)
+        const uint32_t pl = own & 255u, v = own >> 8, axis = pl >> 6, sl = pl & 31u;
+        const uint32_t stride = axis == 0u ? 1u : (uint32_t)kZY;
+        const uint32_t eu = axis == 0u ? kEx + sl * kZY : (axis == 1u ? kEx + sl : kEyT + sl);
+        const uint32_t ends = L.ends[v * kRowWords + pl];
+        const uint32_t u = nth_bit(ends, r);
+        // down to the row where a quad starts at u: u is new there and not
+        // joined to a new cell before it
+        const uint32_t *at = L.avail + v * kRowWords + pl, *eh = L.M + eu + v * stride;
+        const uint32_t bit = 1u << u;
+        uint32_t h1 = 0, cells, joined;  // rows above the last; cells joined to the one below
+        for (;;) {
+          cells = *at;
+          joined = cells & ((cells & *eh) << 1);
+          if ((cells & ~joined & bit) || h1 == v) break;
+          at -= kRowWords;
+          eh -= stride;
+          h1++;
+        }
+        const uint32_t wm1 = (uint32_t)__builtin_ctz(~((joined >> u) >> 1));
+        // pack_quad of (u, v) on the plane's axes
+        const uint32_t su = axis == 2u ? 5u : 0u, sv = axis == 0u ? 5u : 10u;
+        out[k] = ((pl >> 5) << 25) | (sl << (10u - 5u * axis)) | (u << su) | ((v - h1) << sv) |
+                 (wm1 << 15) | (h1 << 20);
+      }
+    }
+    __syncthreads();
+  }
+}
+
 // exclusive scan of one value per lane over the workgroup; returns the total
+template <int T>
 __device__ __forceinline__ uint32_t block_exclusive_scan(MeshLds &L, uint32_t v, uint32_t &excl) {
   const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   uint32_t inc = v;
@@ -656,7 +655,7 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(MeshLds &L, uint32_t v,
   if (lane == 63) L.scan[wave] = inc;
   __syncthreads();
   uint32_t before = 0, total = 0;
-  for (uint32_t w = 0; w < kMeshBlock / 64; w++) {
+  for (uint32_t w = 0; w < T / 64; w++) {
     const uint32_t s = L.scan[w];
     if (w < wave) before += s;
     total += s;
@@ -664,6 +663,37 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(MeshLds &L, uint32_t v,
   excl = before + inc - v;
   __syncthreads();
   return total;
+}
+
+// Counts of the chunk whose masks are in L: the planes' offsets and rows go to
+// L, the chunk's quad count is returned to every thread.
+template <bool GREEDY, int T>
+__device__ __forceinline__ uint32_t chunk_count(LdsOf<GREEDY> &L) {
+  const int t = (int)threadIdx.x;
+  uint32_t occ = 0, mine = 0, excl = 0;
+  if (t < kPlanes) {
+    if constexpr (GREEDY)
+      mine = plane_sweep(L, t, occ);
+    else
+      mine = plane_count(L, t, occ);
+  }
+  const uint32_t total = block_exclusive_scan<T>(L, mine, excl);
+  if (t < kPlanes) {
+    L.pex[t] = excl;
+    L.occ[t] = occ;
+  }
+  return total;
+}
+
+// The counted chunk's quads at out[base ...], up to out[cap]; every thread of
+// the workgroup calls it after a barrier.
+template <bool GREEDY, int T>
+__device__ __forceinline__ void chunk_emit(LdsOf<GREEDY> &L, uint32_t total, uint32_t *out,
+                                           uint64_t base, uint64_t cap) {
+  if constexpr (GREEDY)
+    greedy_emit<T>(L, total, out, base, cap);
+  else
+    culled_emit_balanced<T>(L, total, out, base, cap);
 }
 
 // look-back status word: flag in bits 62-63 (1 = aggregate, 2 = inclusive)
@@ -685,11 +715,11 @@ struct SceneSource {
 
 // SRC 0: packed or dense-grid chunks (meso_chunk_source); 2 / 3: chunks of a
 // brick map / two-level scene
-template <int ES, bool GREEDY, int SRC>
-__global__ void __launch_bounds__(kMeshBlock) mesh_batched_kernel(
+template <int ES, bool GREEDY, int SRC, int T>
+__global__ void __launch_bounds__(T) mesh_batched_kernel(
     meso_chunk_source src, SceneSource ss, uint32_t *counts, uint32_t *prefix, uint32_t *quads,
     uint64_t capacity, unsigned long long *total, MeshWork *work, uint32_t spin_limit) {
-  __shared__ MeshLds L;
+  __shared__ LdsOf<GREEDY> L;
   const int t = (int)threadIdx.x;
   const uint32_t n_chunks = (uint32_t)(SRC == 0 ? src.n_chunks : ss.n_chunks);
   for (;;) {
@@ -698,18 +728,15 @@ __global__ void __launch_bounds__(kMeshBlock) mesh_batched_kernel(
     const uint32_t c = L.chunk;
     if (c >= n_chunks) break;  // uniform: every wave leaves
     if constexpr (SRC == 0) {
-      build_masks<ES>(L, chunk_addr(src, c));
+      build_masks<ES, T>(L, chunk_addr(src, c));
     } else {
       const int32_t nc = (ss.s.n + 31) >> 5;  // a partial last chunk counts
       int32_t cx = ss.xyz[3 * c], cy = ss.xyz[3 * c + 1], cz = ss.xyz[3 * c + 2];
       if (cx < 0 || cy < 0 || cz < 0 || cx >= nc || cy >= nc || cz >= nc)
         cx = cy = cz = nc;  // outside the scene: every brick lookup reads empty
-      build_masks<ES>(L, SceneRows<SRC>{ss.s, cx * 32, cy * 32, cz * 32});
+      build_masks<ES, T>(L, SceneRows<SRC>{ss.s, cx * 32, cy * 32, cz * 32});
     }
-    uint32_t occ = 0;
-    const uint32_t mine = t < kPlanes ? plane_count<GREEDY>(L, t, occ) : 0u;
-    uint32_t excl = 0;
-    const uint32_t chunk_total = block_exclusive_scan(L, mine, excl);
+    const uint32_t chunk_total = chunk_count<GREEDY, T>(L);
     if (t == 0) {
       // publish the aggregate, then add up predecessors until an inclusive one.
       // The value travels inside the status word and no other data is
@@ -754,18 +781,9 @@ __global__ void __launch_bounds__(kMeshBlock) mesh_batched_kernel(
       L.base_lo = (uint32_t)before;
       L.base_hi = (uint32_t)(before >> 32);
     }
-    if constexpr (!GREEDY)
-      if (t < kPlanes) {
-        L.pex[t] = excl;
-        L.occ[t] = occ;
-      }
     __syncthreads();
     const uint64_t base = ((uint64_t)L.base_hi << 32) | L.base_lo;
-    if constexpr (GREEDY) {
-      if (t < kPlanes) plane_emit(L, t, quads, base + excl, capacity, mine);
-    } else {
-      culled_emit_balanced(L, chunk_total, quads, base, capacity);
-    }
+    chunk_emit<GREEDY, T>(L, chunk_total, quads, base, capacity);
     __syncthreads();
   }
 }
@@ -776,11 +794,11 @@ __global__ void __launch_bounds__(kMeshBlock) mesh_batched_kernel(
 // length is read on the device (*n_dev, at most max_n), so that a producer
 // kernel can size it.  Workgroups take chunks from ticket[0]; the last workgroup to leave
 // (ticket[1] counts leavers) sets both back to zero for the next launch.
-template <bool GREEDY, int SRC>
-__global__ void __launch_bounds__(kMeshBlock) mesh_slotted_kernel(
+template <bool GREEDY, int SRC, int T>
+__global__ void __launch_bounds__(T) mesh_slotted_kernel(
     DevScene sc, const int32_t *xyz, const uint32_t *slots, const uint32_t *n_dev, uint32_t max_n,
     uint32_t *slot_count, uint32_t *quads, uint32_t per_slot, unsigned int *ticket) {
-  __shared__ MeshLds L;
+  __shared__ LdsOf<GREEDY> L;
   const int t = (int)threadIdx.x;
   const uint32_t n_chunks = *n_dev < max_n ? *n_dev : max_n;
   const int32_t nc = (sc.n + 31) >> 5;  // a partial last chunk counts
@@ -792,24 +810,13 @@ __global__ void __launch_bounds__(kMeshBlock) mesh_slotted_kernel(
     int32_t cx = xyz[3 * c], cy = xyz[3 * c + 1], cz = xyz[3 * c + 2];
     if (cx < 0 || cy < 0 || cz < 0 || cx >= nc || cy >= nc || cz >= nc)
       cx = cy = cz = nc;  // outside the scene: every brick lookup reads empty
-    build_masks<2>(L, SceneRows<SRC>{sc, cx * 32, cy * 32, cz * 32});
-    uint32_t occ = 0;
-    const uint32_t mine = t < kPlanes ? plane_count<GREEDY>(L, t, occ) : 0u;
-    uint32_t excl = 0;
-    const uint32_t chunk_total = block_exclusive_scan(L, mine, excl);
+    build_masks<2, T>(L, SceneRows<SRC>{sc, cx * 32, cy * 32, cz * 32});
+    const uint32_t chunk_total = chunk_count<GREEDY, T>(L);
     const uint32_t slot = slots[c];
-    const uint64_t base = (uint64_t)slot * per_slot, cap = base + per_slot;
+    const uint64_t base = (uint64_t)slot * per_slot;
     if (t == 0) slot_count[slot] = chunk_total;
-    if constexpr (GREEDY) {
-      if (t < kPlanes) plane_emit(L, t, quads, base + excl, cap, mine);
-    } else {
-      if (t < kPlanes) {
-        L.pex[t] = excl;
-        L.occ[t] = occ;
-      }
-      __syncthreads();
-      culled_emit_balanced(L, chunk_total, quads, base, cap);
-    }
+    __syncthreads();
+    chunk_emit<GREEDY, T>(L, chunk_total, quads, base, base + per_slot);
     __syncthreads();
   }
   if (t == 0 && atomicAdd(&ticket[1], 1u) == gridDim.x - 1u) {
@@ -818,32 +825,20 @@ __global__ void __launch_bounds__(kMeshBlock) mesh_slotted_kernel(
   }
 }
 
-template <int ES, bool GREEDY>
-__global__ void __launch_bounds__(kMeshBlock) mesh_plain_kernel(const void *voxels, uint32_t *count,
-                                                                uint32_t *quads, uint32_t capacity) {
-  __shared__ MeshLds L;
-  const int t = (int)threadIdx.x;
+template <int ES, bool GREEDY, int T>
+__global__ void __launch_bounds__(T) mesh_plain_kernel(const void *voxels, uint32_t *count,
+                                                       uint32_t *quads, uint32_t capacity) {
+  __shared__ LdsOf<GREEDY> L;
   const ChunkAddr a{voxels, 0, 32, 1024};
-  build_masks<ES>(L, a);
-  uint32_t occ = 0;
-  const uint32_t mine = t < kPlanes ? plane_count<GREEDY>(L, t, occ) : 0u;
-  uint32_t excl = 0;
-  const uint32_t chunk_total = block_exclusive_scan(L, mine, excl);
-  if (t == 0) *count = chunk_total;
-  if constexpr (GREEDY) {
-    if (t < kPlanes) plane_emit(L, t, quads, excl, capacity, mine);
-  } else {
-    if (t < kPlanes) {
-      L.pex[t] = excl;
-      L.occ[t] = occ;
-    }
-    __syncthreads();
-    culled_emit_balanced(L, chunk_total, quads, 0, capacity);
-  }
+  build_masks<ES, T>(L, a);
+  const uint32_t chunk_total = chunk_count<GREEDY, T>(L);
+  if (threadIdx.x == 0) *count = chunk_total;
+  __syncthreads();
+  chunk_emit<GREEDY, T>(L, chunk_total, quads, 0, capacity);
 }
 
-template <int ES, bool GREEDY, int SRC>
-static meso_status launch_batched_t(meso_context *ctx, const meso_chunk_source &src,
+template <int ES, bool GREEDY, int SRC, int T>
+static meso_status launch_batched_w(meso_context *ctx, const meso_chunk_source &src,
                                     const SceneSource &ss, int32_t n_chunks, uint32_t *d_counts,
                                     uint32_t *d_prefix, uint32_t *d_quads, uint64_t capacity,
                                     uint64_t *d_total, void *d_work, hipStream_t stream,
@@ -852,19 +847,36 @@ static meso_status launch_batched_t(meso_context *ctx, const meso_chunk_source &
   if (!grid) {
     int per_cu = 0;
     MESO_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &per_cu, mesh_batched_kernel<ES, GREEDY, SRC>, kMeshBlock, 0));
+        &per_cu, mesh_batched_kernel<ES, GREEDY, SRC, T>, T, 0));
     if (per_cu < 1) per_cu = 1;
     grid = per_cu * ctx->props.multiProcessorCount;
   }
   if (grid > n_chunks) grid = n_chunks;
   meso_status st = launch_zero(d_work, meso_mesh_workspace_bytes(n_chunks), stream);
   if (st != MESO_OK) return st;
-  hipLaunchKernelGGL((mesh_batched_kernel<ES, GREEDY, SRC>), dim3(grid), dim3(kMeshBlock), 0,
+  hipLaunchKernelGGL((mesh_batched_kernel<ES, GREEDY, SRC, T>), dim3(grid), dim3(T), 0,
                      stream, src, ss, d_counts, d_prefix, d_quads, capacity,
                      (unsigned long long *)d_total, (MeshWork *)d_work,
                      ctx->lookback_spin_limit);
   MESO_HIP(hipGetLastError());
   return MESO_OK;
+}
+
+// A batch of at most a chunk per CU is bound by one chunk's latency, like a
+// single chunk, and takes the wide workgroups.
+template <int ES, bool GREEDY, int SRC>
+static meso_status launch_batched_t(meso_context *ctx, const meso_chunk_source &src,
+                                    const SceneSource &ss, int32_t n_chunks, uint32_t *d_counts,
+                                    uint32_t *d_prefix, uint32_t *d_quads, uint64_t capacity,
+                                    uint64_t *d_total, void *d_work, hipStream_t stream,
+                                    const MeshLaunch *shape) {
+  if (n_chunks <= ctx->props.multiProcessorCount)
+    return launch_batched_w<ES, GREEDY, SRC, kChunkBlock>(ctx, src, ss, n_chunks, d_counts,
+                                                          d_prefix, d_quads, capacity, d_total,
+                                                          d_work, stream, shape);
+  return launch_batched_w<ES, GREEDY, SRC, GREEDY ? kGreedyBlock : kMeshBlock>(
+      ctx, src, ss, n_chunks, d_counts, d_prefix, d_quads, capacity, d_total, d_work, stream,
+      shape);
 }
 
 // Scratch of meso_mesh_chunks_noalloc: the mesh workspace (ticket, error word
@@ -885,7 +897,10 @@ meso_status init_mesh_scratch(meso_context *ctx) {
   return MESO_OK;
 }
 
-MeshLaunch default_mesh_launch(meso_context *) { return MeshLaunch{kMeshBlock, 0}; }
+int mesh_block(meso_context *ctx, uint32_t mode, int32_t n_chunks) {
+  if (n_chunks <= ctx->props.multiProcessorCount) return kChunkBlock;
+  return mode == MESO_MESH_GREEDY ? kGreedyBlock : kMeshBlock;
+}
 
 static meso_status check_source(const meso_chunk_source *src) {
   MESO_CHECK(src && src->size >= sizeof(meso_chunk_source), MESO_ERR_ARGUMENT_OUT_OF_RANGE,
@@ -954,14 +969,15 @@ static meso_status launch_slotted_t(meso_context *ctx, const meso_scene *scene,
                                     const uint32_t *n_dev, int32_t max_chunks,
                                     uint32_t *slot_count, uint32_t *quads, uint32_t per_slot,
                                     unsigned int *ticket, hipStream_t stream) {
+  constexpr int T = kChunkBlock;
   int per_cu = 0;
   MESO_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &per_cu, mesh_slotted_kernel<GREEDY, SRC>, kMeshBlock, 0));
+      &per_cu, mesh_slotted_kernel<GREEDY, SRC, T>, T, 0));
   if (per_cu < 1) per_cu = 1;
   int grid = per_cu * ctx->props.multiProcessorCount;
   if (grid > max_chunks) grid = max_chunks;
   if (grid < 1) grid = 1;
-  hipLaunchKernelGGL((mesh_slotted_kernel<GREEDY, SRC>), dim3(grid), dim3(kMeshBlock), 0, stream,
+  hipLaunchKernelGGL((mesh_slotted_kernel<GREEDY, SRC, T>), dim3(grid), dim3(T), 0, stream,
                      scene->dev(), xyz, slots, n_dev, (uint32_t)max_chunks, slot_count, quads,
                      per_slot, ticket);
   MESO_HIP(hipGetLastError());
@@ -987,7 +1003,7 @@ meso_status launch_mesh_slotted(meso_context *ctx, const meso_scene *scene, cons
 template <int ES, bool GREEDY>
 static void launch_plain_t(const void *voxels, uint32_t *d_count, uint32_t *d_quads,
                            uint32_t capacity, hipStream_t stream) {
-  hipLaunchKernelGGL((mesh_plain_kernel<ES, GREEDY>), dim3(1), dim3(kMeshBlock), 0, stream, voxels,
+  hipLaunchKernelGGL((mesh_plain_kernel<ES, GREEDY, kChunkBlock>), dim3(1), dim3(kChunkBlock), 0, stream, voxels,
                      d_count, d_quads, capacity);
 }
 

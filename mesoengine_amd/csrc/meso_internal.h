@@ -216,7 +216,8 @@ meso_status launch_mesh_batched(meso_context *ctx, const meso_chunk_source *src,
                                 uint32_t *d_counts, uint32_t *d_prefix, uint32_t *d_quads,
                                 uint64_t capacity, uint64_t *d_total, void *d_work,
                                 hipStream_t stream, const MeshLaunch *shape);
-MeshLaunch default_mesh_launch(meso_context *ctx);
+// threads per workgroup of the batched mesher
+int mesh_block(meso_context *ctx, uint32_t mode, int32_t n_chunks);
 // meshes the first *n_dev chunks of a scene chunk list into fixed slots
 // (quads at slots[c] * per_slot); ticket: 2 counters, zero before the first
 // launch, left at zero by every launch

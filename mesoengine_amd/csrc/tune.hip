@@ -145,7 +145,7 @@ meso_status meso_autotune_mesh(meso_context *ctx, const meso_chunk_source *src, 
   best.best_ms = 1e30f;
   int tried = 0;
   for (int g : grids) {
-    MeshLaunch shape{256, g};
+    MeshLaunch shape{mesh_block(ctx, mode, src->n_chunks), g};
     meso_status st = MESO_OK;
     const float ms = time_ms(
         ctx,
@@ -160,7 +160,7 @@ meso_status meso_autotune_mesh(meso_context *ctx, const meso_chunk_source *src, 
     if (ms < best.best_ms) {
       best.best_ms = ms;
       best.grid = g;
-      best.block = 256;
+      best.block = mesh_block(ctx, mode, src->n_chunks);
       best.variant = g == 0 ? 0 : 1;
     }
   }
