@@ -745,6 +745,7 @@ meso_status meso_scene_create_brickmap_u16(meso_context *ctx, int32_t n, const u
   SCENE_TRY(scene_alloc(ctx, (void **)&sc->masks, (uint64_t)n_bricks * 64, masks, sc));
   SCENE_TRY(scene_alloc(ctx, (void **)&sc->voxels, (uint64_t)n_bricks * 1024, voxels, sc));
   SCENE_TRY(build_coarse(sc, ctx->stream));
+  SCENE_TRY(check_masks(sc, ctx->stream));
   *out = sc;
   return MESO_OK;
 }
@@ -787,6 +788,7 @@ meso_status meso_scene_create_two_level_u16(meso_context *ctx, int32_t n, const 
   SCENE_TRY(scene_alloc(ctx, (void **)&sc->masks, (uint64_t)n_bricks * 64, masks, sc));
   SCENE_TRY(scene_alloc(ctx, (void **)&sc->voxels, (uint64_t)n_bricks * 1024, voxels, sc));
   SCENE_TRY(build_coarse(sc, ctx->stream));
+  SCENE_TRY(check_masks(sc, ctx->stream));
   *out = sc;
   return MESO_OK;
 }

@@ -134,6 +134,9 @@ struct meso_scene {
   // into slots) that holds the brick, 0 when no cell does.
   uint64_t *blocks = nullptr;
   uint32_t *slot_cell = nullptr;
+  // every brick's mask is that of its voxels: so in generated scenes, checked
+  // once for uploaded ones, and kept by every edit and update
+  bool masks_match = false;
   uint16_t *voxels = nullptr;
   uint32_t *top = nullptr;
   uint32_t *occ32 = nullptr;
@@ -205,6 +208,8 @@ meso_status init_mesh_scratch(meso_context *ctx);
 meso_status band_queue(meso_context *ctx, hipStream_t stream, unsigned int **out);
 // builds the empty-space levels (occ32/occ128 or node groups) of a brick scene
 meso_status build_coarse(meso_scene *sc, hipStream_t stream);
+// sets masks_match of a scene whose bricks came from the caller
+meso_status check_masks(meso_scene *sc, hipStream_t stream);
 void free_scene_arrays(meso_scene *sc);
 
 // kernels launched by other translation units
