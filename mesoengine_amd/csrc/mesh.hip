@@ -791,11 +791,10 @@ __global__ void __launch_bounds__(T) mesh_slotted_kernel(
   const int t = (int)threadIdx.x;
   const uint32_t n_chunks = *n_dev < max_n ? *n_dev : max_n;
   const int32_t nc = (sc.n + 31) >> 5;  // a partial last chunk counts
-  for (;;) {
-    if (t == 0) L.chunk = atomicAdd(&ticket[0], 1u);
-    __syncthreads();
-    const uint32_t c = L.chunk;
-    if (c >= n_chunks) break;  // uniform: every wave leaves
+  // the first chunk is the workgroup's own; tickets, an add to one word that
+  // takes 50 to 100 ns of its time each, hand out the rest
+  const bool tickets = n_chunks > gridDim.x;
+  for (uint32_t c = blockIdx.x; c < n_chunks;) {  // uniform: every wave leaves
     int32_t cx = xyz[3 * c], cy = xyz[3 * c + 1], cz = xyz[3 * c + 2];
     if (cx < 0 || cy < 0 || cz < 0 || cx >= nc || cy >= nc || cz >= nc)
       cx = cy = cz = nc;  // outside the scene: every brick lookup reads empty
@@ -806,9 +805,13 @@ __global__ void __launch_bounds__(T) mesh_slotted_kernel(
     if (t == 0) slot_count[slot] = chunk_total;
     __syncthreads();
     chunk_emit<GREEDY, T>(L, chunk_total, quads, base, base + per_slot);
+    if (!tickets) break;
+    if (t == 0) L.chunk = atomicAdd(&ticket[0], 1u);
+    __syncthreads();
+    c = gridDim.x + L.chunk;
     __syncthreads();
   }
-  if (t == 0 && atomicAdd(&ticket[1], 1u) == gridDim.x - 1u) {
+  if (tickets && t == 0 && atomicAdd(&ticket[1], 1u) == gridDim.x - 1u) {
     __hip_atomic_store(&ticket[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(&ticket[1], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }

@@ -37,6 +37,12 @@ enum : int {
   kCntWords = 16
 };
 
+// the camera of one update: its chunk and unit forward vector
+struct PoolView3 {
+  int32_t c[3];
+  float f[3];
+};
+
 struct PoolGeom {
   int32_t R, RB;       // forward / backward radius, chunks
   float thr;           // view-cone threshold
@@ -118,108 +124,243 @@ __global__ void pool_begin_kernel(uint32_t *counters, uint32_t limit) {
   counters[kCntStamp] = counters[kCntStamp] + 1u;
 }
 
-// Candidate keys: importance descending (complemented float bits;
-// importances are positive), then chunk index.  With `compact` the
-// candidates are appended to `keys` in any order (their number is the
-// candidate counter); otherwise there is one key per offset of the
-// (2R+1)^3 cube and offsets that are no candidate get the largest key, so
-// that a full sort puts them last.
+// Key of the cube's offset k when its chunk is a candidate (desired, inside the
+// scene, not empty, not resident), else ~0: importance descending
+// (complemented float bits; importances are positive), then chunk index.
 template <int KIND>
-__global__ void __launch_bounds__(256) pool_rank_kernel(DevScene s, PoolGeom g, int32_t cx0,
-                                                        int32_t cy0, int32_t cz0, float f0,
-                                                        float f1, float f2,
-                                                        const uint32_t *lookup, uint64_t *keys,
-                                                        uint64_t cube, uint32_t *counters,
-                                                        bool compact) {
-  const uint64_t k = block_id() * 256u + threadIdx.x;
-  bool cand = false;
-  uint64_t key = ~0ull;
-  if (k < cube) {
-    const uint32_t side = (uint32_t)g.side;
-    const int32_t dx = (int32_t)(k % side) - g.R, dy = (int32_t)((k / side) % side) - g.R,
-                  dz = (int32_t)(k / ((uint64_t)side * side)) - g.R;
-    const int32_t cx = cx0 + dx, cy = cy0 + dy, cz = cz0 + dz;
-    if (cx >= 0 && cy >= 0 && cz >= 0 && cx < g.nc && cy < g.nc && cz < g.nc) {
-      const uint32_t idx = (uint32_t)cx + (uint32_t)g.nc * ((uint32_t)cy + (uint32_t)g.nc * (uint32_t)cz);
-      if (lookup[idx] == kNoSlot && chunk_desired(dx, dy, dz, f0, f1, f2, g) &&
-          chunk_nonempty<KIND>(s, g.nc, cx, cy, cz)) {
-        const float imp = chunk_importance(dx, dy, dz, f0, f1, f2);
-        key = ((uint64_t)(~__float_as_uint(imp)) << 32) | idx;
-        cand = true;
-      }
-    }
-    if (!compact) keys[k] = key;
-  }
-  const uint64_t b = __ballot(cand);
-  const uint32_t lane = threadIdx.x & 63u;
-  uint32_t base = 0u;
-  if (lane == 0u && b) base = atomicAdd(&counters[kCntCandidates], (uint32_t)__popcll(b));
-  if (compact) {
-    base = (uint32_t)__builtin_amdgcn_readlane((int)base, 0);
-    if (cand) keys[base + (uint32_t)__popcll(b & ((1ull << lane) - 1ull))] = key;
-  }
+__device__ __forceinline__ uint64_t candidate_key(const DevScene &s, const PoolGeom &g,
+                                                  const PoolView3 &v, const uint32_t *lookup,
+                                                  uint32_t k) {
+  const uint32_t side = (uint32_t)g.side;
+  const int32_t dx = (int32_t)(k % side) - g.R, dy = (int32_t)((k / side) % side) - g.R,
+                dz = (int32_t)(k / (side * side)) - g.R;
+  const int32_t cx = v.c[0] + dx, cy = v.c[1] + dy, cz = v.c[2] + dz;
+  if (cx < 0 || cy < 0 || cz < 0 || cx >= g.nc || cy >= g.nc || cz >= g.nc) return ~0ull;
+  const uint32_t idx = (uint32_t)cx + (uint32_t)g.nc * ((uint32_t)cy + (uint32_t)g.nc * (uint32_t)cz);
+  if (lookup[idx] != kNoSlot || !chunk_desired(dx, dy, dz, v.f[0], v.f[1], v.f[2], g) ||
+      !chunk_nonempty<KIND>(s, g.nc, cx, cy, cz))
+    return ~0ull;
+  const float imp = chunk_importance(dx, dy, dz, v.f[0], v.f[1], v.f[2]);
+  return ((uint64_t)(~__float_as_uint(imp)) << 32) | idx;
 }
 
-// Victim keys, one per slot: free slots first (by slot), then resident
-// chunks by importance under this camera (ascending), then slot.
-__global__ void __launch_bounds__(256) pool_victim_kernel(PoolGeom g, int32_t cx0, int32_t cy0,
-                                                          int32_t cz0, float f0, float f1,
-                                                          float f2, const uint32_t *slot_chunk,
-                                                          uint64_t *keys) {
-  const uint32_t sl = (uint32_t)(block_id() * 256u + threadIdx.x);
-  if (sl >= (uint32_t)g.capacity) return;
+// Key of a slot as a victim: free slots first (by slot), then resident chunks
+// by importance under this camera (ascending), then slot.
+__device__ __forceinline__ uint64_t victim_key(const PoolGeom &g, const PoolView3 &v,
+                                               const uint32_t *slot_chunk, uint32_t sl) {
   const uint32_t c = slot_chunk[sl];
-  if (c == kNoSlot) {
-    keys[sl] = sl;
-    return;
-  }
+  if (c == kNoSlot) return sl;
   const uint32_t nc = (uint32_t)g.nc;
   const int32_t x = (int32_t)(c % nc), y = (int32_t)((c / nc) % nc), z = (int32_t)(c / (nc * nc));
-  const float imp = chunk_importance(x - cx0, y - cy0, z - cz0, f0, f1, f2);
-  keys[sl] = ((uint64_t)__float_as_uint(imp) << 32) | sl;
+  const float imp = chunk_importance(x - v.c[0], y - v.c[1], z - v.c[2], v.f[0], v.f[1], v.f[2]);
+  return ((uint64_t)__float_as_uint(imp) << 32) | sl;
+}
+
+// For the full sorts: one key per offset of the cube (offsets that are no
+// candidate get the largest key, which the sort puts last) ...
+template <int KIND>
+__global__ void __launch_bounds__(256) pool_rank_kernel(DevScene s, PoolGeom g, PoolView3 v,
+                                                        const uint32_t *lookup, uint64_t *keys,
+                                                        uint32_t cube, uint32_t *counters) {
+  const uint32_t k = blockIdx.x * 256u + threadIdx.x;
+  const uint64_t key = k < cube ? candidate_key<KIND>(s, g, v, lookup, k) : ~0ull;
+  if (k < cube) keys[k] = key;
+  const uint64_t b = __ballot(key != ~0ull);
+  if ((threadIdx.x & 63u) == 0u && b) atomicAdd(&counters[kCntCandidates], (uint32_t)__popcll(b));
+}
+
+// ... and one per slot.
+__global__ void __launch_bounds__(256) pool_victim_kernel(PoolGeom g, PoolView3 v,
+                                                          const uint32_t *slot_chunk,
+                                                          uint64_t *keys) {
+  const uint32_t sl = blockIdx.x * 256u + threadIdx.x;
+  if (sl < (uint32_t)g.capacity) keys[sl] = victim_key(g, v, slot_chunk, sl);
+}
+
+// Bins of keys, monotone in the key.  By importance: 256 bins per power of two
+// from 1/8 to 64 (importances lie in [3/16, 64] and at 1e6), clamped outside.
+// The free slots among the victims come first, 256 bins of them by slot.
+constexpr uint32_t kBins = 4096u, kFreeBins = 256u;
+__device__ __forceinline__ uint32_t importance_bin(uint32_t bits) {
+  constexpr uint32_t base = 0x3E000000u >> 15;  // 1/8
+  const uint32_t q = bits >> 15;
+  const uint32_t b = q <= base ? 0u : q - base;
+  return b < kBins - kFreeBins ? b : kBins - kFreeBins - 1u;
+}
+__device__ __forceinline__ uint32_t key_bin(uint64_t key, bool victim, uint32_t capacity) {
+  const uint32_t hi = (uint32_t)(key >> 32);
+  if (!victim) return kBins - 1u - importance_bin(~hi);
+  if (hi) return kFreeBins + importance_bin(hi);
+  const uint32_t bits = capacity > 1u ? 32u - (uint32_t)__builtin_clz(capacity - 1u) : 0u;
+  return (uint32_t)key >> (bits > 8u ? bits - 8u : 0u);
+}
+
+// What the select keeps between its kernels, zero between updates: candidates
+// per segment (one counter per 64 bytes: adds to one word take 50 to 100 ns
+// each, whoever adds), a count of finished lists, and the lists' bins.
+constexpr uint32_t kSegs = 8u;
+struct SelectState {
+  uint32_t seg[kSegs * 16u];
+  uint32_t done, pad[15];
+  uint32_t bins[2][kBins];
+};
+
+// Keys for the select: the first rank_blocks workgroups append the candidates
+// of 1024 offsets each to segment blockIdx % 8 of the list (in any order), the
+// others write the victims' keys.  Each counts its keys' bins.
+constexpr uint32_t kKeyThreads = 1024u;
+template <int KIND>
+__global__ void __launch_bounds__(kKeyThreads)
+    pool_keys_kernel(DevScene s, PoolGeom g, PoolView3 v, const uint32_t *lookup,
+                     const uint32_t *slot_chunk, uint32_t cube, uint32_t rank_blocks,
+                     uint32_t seg_cap, uint64_t *cand, uint64_t *vict, SelectState *st) {
+  __shared__ uint32_t bins[kBins];
+  __shared__ uint32_t wave_n[kKeyThreads / 64u], base;
+  const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+  const bool victims = blockIdx.x >= rank_blocks;
+  for (uint32_t i = t; i < kBins; i += kKeyThreads) bins[i] = 0u;
+  uint64_t key = ~0ull;
+  bool take = false;
+  if (victims) {
+    const uint32_t sl = (blockIdx.x - rank_blocks) * kKeyThreads + t;
+    take = sl < (uint32_t)g.capacity;
+    if (take) {
+      key = victim_key(g, v, slot_chunk, sl);
+      vict[sl] = key;
+    }
+  } else {
+    const uint32_t k = blockIdx.x * kKeyThreads + t;
+    if (k < cube) key = candidate_key<KIND>(s, g, v, lookup, k);
+    take = key != ~0ull;
+  }
+  const uint64_t b = __ballot(take);
+  if (lane == 0u) wave_n[wave] = (uint32_t)__popcll(b);
+  __syncthreads();
+  if (take) atomicAdd(&bins[key_bin(key, victims, (uint32_t)g.capacity)], 1u);
+  if (!victims) {
+    uint32_t at = 0, all = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kKeyThreads / 64u; w++) {
+      at += w < wave ? wave_n[w] : 0u;
+      all += wave_n[w];
+    }
+    const uint32_t seg = blockIdx.x % kSegs;
+    if (t == 0u) base = all ? atomicAdd(&st->seg[seg * 16u], all) : 0u;
+    __syncthreads();
+    if (take)
+      cand[(uint64_t)seg * seg_cap + base + at + (uint32_t)__popcll(b & ((1ull << lane) - 1ull))] = key;
+  }
+  __syncthreads();
+  for (uint32_t i = t; i < kBins; i += kKeyThreads)
+    if (bins[i]) atomicAdd(&st->bins[victims ? 1 : 0][i], bins[i]);
+}
+
+// Candidate i takes victim i when the victim is free or strictly less
+// important.  Candidates descend and victims ascend in importance, so the
+// pairs that qualify are a prefix; its length is the first failure.
+__device__ __forceinline__ bool pair_qualifies(uint64_t ck, uint64_t vk) {
+  if (ck == ~0ull) return false;
+  if ((uint32_t)(vk >> 32) == 0u) return true;
+  const float ci = __uint_as_float(~(uint32_t)(ck >> 32));
+  const float vi = __uint_as_float((uint32_t)(vk >> 32));
+  return vi < ci;
+}
+
+// Applies pair i: the victim's chunk leaves the lookup table, the candidate
+// takes its slot, and the load list for the mesher is written.  Old chunks
+// (resident) and new ones (not resident) are disjoint sets and every pair has
+// its own slot, so the writes never collide.  True when a chunk was evicted.
+struct PoolTables {
+  int32_t nc;
+  uint32_t *lookup, *slot_chunk, *slot_stamp;
+  int32_t *load_xyz;
+  uint32_t *load_slot;
+};
+__device__ __forceinline__ bool apply_pair(const PoolTables &p, uint32_t i, uint64_t ck,
+                                           uint64_t vk, uint32_t stamp) {
+  const uint32_t sl = (uint32_t)vk, c = (uint32_t)ck, n = (uint32_t)p.nc;
+  const uint32_t old = p.slot_chunk[sl];
+  if (old != kNoSlot) p.lookup[old] = kNoSlot;
+  p.lookup[c] = sl;
+  p.slot_chunk[sl] = c;
+  p.slot_stamp[sl] = stamp;
+  p.load_xyz[3 * i] = (int32_t)(c % n);
+  p.load_xyz[3 * i + 1] = (int32_t)((c / n) % n);
+  p.load_xyz[3 * i + 2] = (int32_t)(c / (n * n));
+  p.load_slot[i] = sl;
+  return old != kNoSlot;
 }
 
 // The first `limit` keys of a list in ascending order, for limits up to
-// kSelMax: one workgroup per list, block 0 the compact candidates (their
-// number is the candidate counter), block 1 the victims (one per slot).
-// An MSB-first radix select over 8-bit digits finds t, the limit-th
-// smallest key: per digit a histogram in LDS of the keys that share the
-// digits found so far, and a scan by one wave; once at most kSelSmall keys
-// share them, one wave ranks those keys directly.  The keys below t are
-// gathered into LDS, the remaining places up to the limit take t, and a
-// bitonic sort orders the kpad (power of two >= limit) places.  That is
-// the first `limit` places of a full sort of the list, repeated keys
-// included.  A list no longer than the limit is taken whole and padded
-// with the largest key, which is what a full sort of the cube's keys puts
-// after the candidates.  The first kSelPer * kSelThreads keys stay in
+// kSelMax, then the pairing.  One workgroup per list, block 0 the candidates,
+// block 1 the victims (one per slot).  The keys' bins, counted when the keys
+// were made, name the bin that holds t, the limit-th smallest key.  Where the
+// keys up to that bin are at most one per thread, they are gathered into LDS
+// bin by bin and a thread counts the keys before its own in its bin, which is
+// its place.  (A radix select and a bitonic sort took three to four passes
+// over the list and 20 barriers: 37 us against 20 for 256 of 16,384 slots and
+// 15,000 candidates, pairing included.)
+// Otherwise (limits near and above the threads) an MSB-first radix select over 8-bit digits finds t: per digit a histogram in
+// LDS of the keys that share the digits found so far, and a scan by one wave;
+// once at most kSelSmall keys share them, one wave ranks those keys directly.
+// The keys below t are gathered into LDS, the remaining places up to the limit
+// take t, and a bitonic sort orders the kpad (power of two >= limit) places.
+// Either way that is the first `limit` places of a full sort of the list,
+// repeated keys included.  A list no longer than the limit is taken whole and
+// padded with the largest key, which is what a full sort of the cube's keys
+// puts after the candidates.  The first kSelPer * kSelThreads keys stay in
 // registers across the passes; the rest are re-read from memory.
+// The list that is finished last pairs both and applies the pairs.
 constexpr uint32_t kSelThreads = 1024u, kSelMax = 4096u, kSelPer = 16u, kSelSmall = 64u;
 // Longest list the one-workgroup select takes: keys past the first
-// kSelPer * kSelThreads are re-read on every radix pass, so past eight times
+// kSelPer * kSelThreads are re-read on every pass, so past eight times
 // that the device-wide radix sorts are faster.
 constexpr uint64_t kSelListMax = 8ull * kSelPer * kSelThreads;
 
 __global__ void __launch_bounds__(kSelThreads)
-    pool_select_kernel(const uint64_t *cand, const uint64_t *vict, uint32_t cap, uint32_t limit,
-                       uint32_t kpad, const uint32_t *counters, uint64_t *cand_out,
-                       uint64_t *vict_out) {
+    pool_select_kernel(const uint64_t *cand, const uint64_t *vict, uint32_t cap, uint32_t seg_cap,
+                       uint32_t limit, uint32_t kpad, SelectState *st, uint64_t *cand_out,
+                       uint64_t *vict_out, PoolTables tab, uint32_t *counters) {
   __shared__ uint64_t buf[kSelMax];
   __shared__ uint32_t hist[256];
   __shared__ uint32_t spread_hist[16 * 257];  // 16 copies, by lane, for the top two digits
-  __shared__ uint32_t s_bin, s_below, s_cnt, s_fill;
+  __shared__ __attribute__((aligned(16))) uint32_t fill[kBins];  // next place of each bin
+  __shared__ uint32_t s_bin, s_below, s_cnt, s_fill, s_wave[kSelThreads / 64u];
   __shared__ uint64_t s_key;
-  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const bool victims = blockIdx.x != 0u;
-  const uint64_t *keys = victims ? vict : cand;
   uint64_t *out = victims ? vict_out : cand_out;
-  const uint32_t n = victims ? cap : counters[kCntCandidates];
+  // places of the candidates' segments in the list
+  uint32_t seg_end[kSegs], n = 0;
+#pragma unroll
+  for (uint32_t j = 0; j < kSegs; j++) {
+    n += victims ? 0u : st->seg[j * 16u];
+    seg_end[j] = n;
+  }
+  n = victims ? cap : n;
+  const auto key_at = [&](uint32_t i) {
+    if (victims) return vict[i];
+    uint32_t seg = 0, first = 0;
+#pragma unroll
+    for (uint32_t j = 0; j + 1u < kSegs; j++) {
+      const bool past = i >= seg_end[j];
+      seg += past ? 1u : 0u;
+      first = past ? seg_end[j] : first;
+    }
+    return cand[(uint64_t)seg * seg_cap + (i - first)];
+  };
   constexpr uint32_t kHeld = kSelPer * kSelThreads;
   uint64_t r[kSelPer];
 #pragma unroll
   for (uint32_t j = 0; j < kSelPer; j++) {
     const uint32_t i = tid + j * kSelThreads;
-    r[j] = i < n ? keys[i] : 0ull;
+    r[j] = i < n ? key_at(i) : 0ull;
   }
+  // this list's bins, four per thread, which go back to zero for the next update
+  uint4 *bins = (uint4 *)st->bins[victims ? 1 : 0];
+  const uint4 h4 = bins[tid];
+  bins[tid] = make_uint4(0u, 0u, 0u, 0u);
+  const auto bin_of = [&](uint64_t key) { return key_bin(key, victims, cap); };
   // f(key, valid) for every key of the list; each call is made by all lanes
   // of the workgroup together, so f may use wave-wide operations
   auto each = [&](auto &&f) {
@@ -227,215 +368,278 @@ __global__ void __launch_bounds__(kSelThreads)
     for (uint32_t j = 0; j < kSelPer; j++) f(r[j], tid + j * kSelThreads < n);
     for (uint32_t b = kHeld; b < n; b += kSelThreads) {
       const uint32_t i = b + tid;
-      f(i < n ? keys[i] : 0ull, i < n);
+      f(i < n ? key_at(i) : 0ull, i < n);
     }
   };
-  uint64_t t = ~0ull;     // the limit-th smallest key
-  uint32_t rem = limit;   // its rank among the keys sharing the digits found
-  uint32_t less = 0u;     // keys sharing them that are below t
-  if (n > limit) {
-    uint64_t prefix = 0ull, hi = 0ull;  // digits found, and their bits
-    int shift = 56;
-    bool small = false;
-    for (;; shift -= 8) {
-      // The top digits are shared by most keys of a wave; lanes that add to
-      // one LDS word serialize, so those passes count into 16 copies
-      // (lane & 15, stride 257 words) that are summed afterwards.
-      const bool spread = shift >= 48;
-      if (tid < 256u) hist[tid] = 0u;
-      if (spread)
-        for (uint32_t i = tid; i < 16u * 257u; i += kSelThreads) spread_hist[i] = 0u;
-      __syncthreads();
-      each([&](uint64_t key, bool valid) {
-        const bool m = valid && (key & hi) == prefix;
-        const uint32_t d = (uint32_t)(key >> shift) & 255u;
-        if (m) atomicAdd(spread ? &spread_hist[(lane & 15u) * 257u + d] : &hist[d], 1u);
-      });
-      __syncthreads();
-      if (spread) {
-        if (tid < 256u) {
-          uint32_t acc = 0u;
+  const uint64_t *sorted = buf;
+  uint32_t held = limit;  // places of `sorted`; the largest key behind them
+  // the bins' first places; the bin in which the running count reaches the
+  // limit, and the keys up to its end
+  const uint32_t mine = h4.x + h4.y + h4.z + h4.w;
+  uint32_t inc = mine;
 #pragma unroll
-          for (uint32_t c = 0; c < 16u; c++) acc += spread_hist[c * 257u + tid];
-          hist[tid] = acc;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t v = __shfl_up(inc, o);
+    if ((int)lane >= o) inc += v;
+  }
+  if (lane == 63u) s_wave[wave] = inc;
+  if (tid == 0u) {
+    s_bin = kBins - 1u;
+    s_cnt = n;
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t w = 0; w < kSelThreads / 64u; w++) inc += w < wave ? s_wave[w] : 0u;
+  const uint32_t c0 = inc - mine, c1 = c0 + h4.x, c2 = c1 + h4.y, c3 = c2 + h4.z;
+  ((uint4 *)fill)[tid] = make_uint4(c0, c1, c2, c3);
+  if (inc >= limit && c0 < limit) {  // one thread, if the list reaches the limit
+    s_bin = 4u * tid + (c1 >= limit ? 0u : c2 >= limit ? 1u : c3 >= limit ? 2u : 3u);
+    s_cnt = c1 >= limit ? c1 : c2 >= limit ? c2 : c3 >= limit ? c3 : inc;
+  }
+  __syncthreads();
+  const uint32_t t_bin = s_bin, m = s_cnt;
+  __syncthreads();
+  if (m <= kSelThreads) {  // uniform
+    // the keys up to t_bin, bin by bin; fill[bin] then is the bin's end
+    each([&](uint64_t key, bool valid) {
+      const uint32_t bin = bin_of(key);
+      if (valid && bin <= t_bin) buf[atomicAdd(&fill[bin], 1u)] = key;
+    });
+    __syncthreads();
+    uint64_t *placed = buf + kSelThreads;
+    if (tid < m) {
+      const uint64_t k = buf[tid];
+      const uint32_t bin = bin_of(k), lo = bin ? fill[bin - 1u] : 0u, hi = fill[bin];
+      uint32_t rank = lo;
+      for (uint32_t j = lo; j < hi; j++) {
+        const uint64_t o = buf[j];
+        rank += (o < k || (o == k && j < tid)) ? 1u : 0u;
+      }
+      placed[rank] = k;
+    }
+    sorted = placed;
+    held = m;
+  } else {
+    uint64_t t = ~0ull;     // the limit-th smallest key
+    uint32_t rem = limit;   // its rank among the keys sharing the digits found
+    uint32_t less = 0u;     // keys sharing them that are below t
+    if (n > limit) {
+      uint64_t prefix = 0ull, hi = 0ull;  // digits found, and their bits
+      int shift = 56;
+      bool small = false;
+      for (;; shift -= 8) {
+        // The top digits are shared by most keys of a wave; lanes that add to
+        // one LDS word serialize, so those passes count into 16 copies
+        // (lane & 15, stride 257 words) that are summed afterwards.
+        const bool spread = shift >= 48;
+        if (tid < 256u) hist[tid] = 0u;
+        if (spread)
+          for (uint32_t i = tid; i < 16u * 257u; i += kSelThreads) spread_hist[i] = 0u;
+        __syncthreads();
+        each([&](uint64_t key, bool valid) {
+          const bool m = valid && (key & hi) == prefix;
+          const uint32_t d = (uint32_t)(key >> shift) & 255u;
+          if (m) atomicAdd(spread ? &spread_hist[(lane & 15u) * 257u + d] : &hist[d], 1u);
+        });
+        __syncthreads();
+        if (spread) {
+          if (tid < 256u) {
+            uint32_t acc = 0u;
+  #pragma unroll
+            for (uint32_t c = 0; c < 16u; c++) acc += spread_hist[c * 257u + tid];
+            hist[tid] = acc;
+          }
+          __syncthreads();
+        }
+        if (tid < 64u) {
+          const uint32_t h0 = hist[4u * tid], h1 = hist[4u * tid + 1u], h2 = hist[4u * tid + 2u],
+                         h3 = hist[4u * tid + 3u];
+          const uint32_t c = h0 + h1 + h2 + h3;
+          uint32_t inc = c;
+  #pragma unroll
+          for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t v = __shfl_up(inc, o);
+            if ((int)tid >= o) inc += v;
+          }
+          // the bins hold at least rem keys in all, so some lane reaches rem
+          const uint64_t over = __ballot(inc >= rem);
+          const uint32_t at = over ? (uint32_t)__ffsll((long long)over) - 1u : 63u;
+          if (tid == at) {
+            uint32_t cum = inc - c, bin = 4u * tid, hb = h0;
+            if (cum + h0 < rem) {
+              cum += h0, bin++, hb = h1;
+              if (cum + h1 < rem) {
+                cum += h1, bin++, hb = h2;
+                if (cum + h2 < rem) cum += h2, bin++, hb = h3;
+              }
+            }
+            s_bin = bin;
+            s_below = cum;
+            s_cnt = hb;
+          }
         }
         __syncthreads();
-      }
-      if (tid < 64u) {
-        const uint32_t h0 = hist[4u * tid], h1 = hist[4u * tid + 1u], h2 = hist[4u * tid + 2u],
-                       h3 = hist[4u * tid + 3u];
-        const uint32_t c = h0 + h1 + h2 + h3;
-        uint32_t inc = c;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-          const uint32_t v = __shfl_up(inc, o);
-          if ((int)tid >= o) inc += v;
+        prefix |= (uint64_t)s_bin << shift;
+        hi |= 255ull << shift;
+        rem -= s_below;
+        if (s_cnt <= kSelSmall) {
+          small = true;
+          break;
         }
-        // the bins hold at least rem keys in all, so some lane reaches rem
-        const uint64_t over = __ballot(inc >= rem);
-        const uint32_t at = over ? (uint32_t)__ffsll((long long)over) - 1u : 63u;
-        if (tid == at) {
-          uint32_t cum = inc - c, bin = 4u * tid, hb = h0;
-          if (cum + h0 < rem) {
-            cum += h0, bin++, hb = h1;
-            if (cum + h1 < rem) {
-              cum += h1, bin++, hb = h2;
-              if (cum + h2 < rem) cum += h2, bin++, hb = h3;
-            }
+        if (shift == 0) break;
+      }
+      if (small) {
+        // few keys hold the digits found: gather them, and one wave ranks
+        // them (ties by place); the key of rank rem - 1 is t
+        if (tid == 0u) s_fill = 0u;
+        __syncthreads();
+        each([&](uint64_t key, bool valid) {
+          if (valid && (key & hi) == prefix) {
+            const uint32_t pos = atomicAdd(&s_fill, 1u);
+            if (pos < kSelSmall) buf[pos] = key;
           }
-          s_bin = bin;
-          s_below = cum;
-          s_cnt = hb;
+        });
+        __syncthreads();
+        const uint32_t cnt = s_cnt;
+        if (tid < cnt) {
+          const uint64_t k = buf[tid];
+          uint32_t rank = 0u, lt = 0u;
+          for (uint32_t j = 0; j < cnt; j++) {
+            const uint64_t o = buf[j];
+            lt += o < k ? 1u : 0u;
+            rank += (o < k || (o == k && j < tid)) ? 1u : 0u;
+          }
+          if (rank == rem - 1u) {
+            s_key = k;
+            s_fill = lt;
+          }
         }
-      }
-      __syncthreads();
-      prefix |= (uint64_t)s_bin << shift;
-      hi |= 255ull << shift;
-      rem -= s_below;
-      if (s_cnt <= kSelSmall) {
-        small = true;
-        break;
-      }
-      if (shift == 0) break;
-    }
-    if (small) {
-      // few keys hold the digits found: gather them, and one wave ranks
-      // them (ties by place); the key of rank rem - 1 is t
-      if (tid == 0u) s_fill = 0u;
-      __syncthreads();
-      each([&](uint64_t key, bool valid) {
-        if (valid && (key & hi) == prefix) {
-          const uint32_t pos = atomicAdd(&s_fill, 1u);
-          if (pos < kSelSmall) buf[pos] = key;
-        }
-      });
-      __syncthreads();
-      const uint32_t cnt = s_cnt;
-      if (tid < cnt) {
-        const uint64_t k = buf[tid];
-        uint32_t rank = 0u, lt = 0u;
-        for (uint32_t j = 0; j < cnt; j++) {
-          const uint64_t o = buf[j];
-          lt += o < k ? 1u : 0u;
-          rank += (o < k || (o == k && j < tid)) ? 1u : 0u;
-        }
-        if (rank == rem - 1u) {
-          s_key = k;
-          s_fill = lt;
-        }
-      }
-      __syncthreads();
-      t = s_key;
-      less = s_fill;
-      __syncthreads();  // s_fill is reset for the gather below
-    } else {
-      t = prefix;  // every key holding all eight digits equals t
-    }
-  }
-  // keys below t: n when the list is taken whole, else the keys under the
-  // digits' bin plus those of the small set below t
-  const uint32_t below = n > limit ? limit - rem + less : n;
-  if (tid == 0u) s_fill = 0u;
-  for (uint32_t i = below + tid; i < kpad; i += kSelThreads) buf[i] = i < limit ? t : ~0ull;
-  __syncthreads();
-  each([&](uint64_t key, bool valid) {
-    const bool m = valid && key < t;
-    const uint64_t mb = __ballot(m);
-    if (!mb) return;
-    uint32_t base = 0u;
-    if (lane == 0u) base = atomicAdd(&s_fill, (uint32_t)__popcll(mb));
-    base = (uint32_t)__builtin_amdgcn_readlane((int)base, 0);
-    const uint32_t pos = base + (uint32_t)__popcll(mb & ((1ull << lane) - 1ull));
-    if (m && pos < below) buf[pos] = key;
-  });
-  // bitonic sort, two layers (strides s and s/2) per barrier where the
-  // stage has them: a thread orders the four places i, i + s/2, i + s,
-  // i + 3s/2 in registers
-  for (uint32_t size = 2u; size <= kpad; size <<= 1) {
-    for (uint32_t stride = size >> 1; stride > 0u;) {
-      __syncthreads();
-      if (stride >= 2u) {
-        const uint32_t h = stride >> 1, p1 = (uint32_t)__ffs((int)h) - 1u;
-        for (uint32_t q = tid; q < kpad / 4u; q += kSelThreads) {
-          const uint32_t i = ((q >> p1) << (p1 + 2u)) | (q & (h - 1u));
-          const bool up = (i & size) == 0u;
-          uint64_t a0 = buf[i], a1 = buf[i + h], a2 = buf[i + stride], a3 = buf[i + stride + h];
-          auto order = [up](uint64_t &x, uint64_t &y) {
-            if ((x > y) == up) {
-              const uint64_t z = x;
-              x = y;
-              y = z;
-            }
-          };
-          order(a0, a2);
-          order(a1, a3);
-          order(a0, a1);
-          order(a2, a3);
-          buf[i] = a0;
-          buf[i + h] = a1;
-          buf[i + stride] = a2;
-          buf[i + stride + h] = a3;
-        }
-        stride >>= 2;
+        __syncthreads();
+        t = s_key;
+        less = s_fill;
+        __syncthreads();  // s_fill is reset for the gather below
       } else {
-        for (uint32_t q = tid; q < kpad / 2u; q += kSelThreads) {
-          const uint32_t i = 2u * q;
-          const uint64_t a = buf[i], b = buf[i + 1u];
-          if ((a > b) == ((i & size) == 0u)) {
-            buf[i] = b;
-            buf[i + 1u] = a;
+        t = prefix;  // every key holding all eight digits equals t
+      }
+    }
+    // keys below t: n when the list is taken whole, else the keys under the
+    // digits' bin plus those of the small set below t
+    const uint32_t below = n > limit ? limit - rem + less : n;
+    if (tid == 0u) s_fill = 0u;
+    for (uint32_t i = below + tid; i < kpad; i += kSelThreads) buf[i] = i < limit ? t : ~0ull;
+    __syncthreads();
+    each([&](uint64_t key, bool valid) {
+      const bool m = valid && key < t;
+      const uint64_t mb = __ballot(m);
+      if (!mb) return;
+      uint32_t base = 0u;
+      if (lane == 0u) base = atomicAdd(&s_fill, (uint32_t)__popcll(mb));
+      base = (uint32_t)__builtin_amdgcn_readlane((int)base, 0);
+      const uint32_t pos = base + (uint32_t)__popcll(mb & ((1ull << lane) - 1ull));
+      if (m && pos < below) buf[pos] = key;
+    });
+    // bitonic sort, two layers (strides s and s/2) per barrier where the
+    // stage has them: a thread orders the four places i, i + s/2, i + s,
+    // i + 3s/2 in registers
+    for (uint32_t size = 2u; size <= kpad; size <<= 1) {
+      for (uint32_t stride = size >> 1; stride > 0u;) {
+        __syncthreads();
+        if (stride >= 2u) {
+          const uint32_t h = stride >> 1, p1 = (uint32_t)__ffs((int)h) - 1u;
+          for (uint32_t q = tid; q < kpad / 4u; q += kSelThreads) {
+            const uint32_t i = ((q >> p1) << (p1 + 2u)) | (q & (h - 1u));
+            const bool up = (i & size) == 0u;
+            uint64_t a0 = buf[i], a1 = buf[i + h], a2 = buf[i + stride], a3 = buf[i + stride + h];
+            auto order = [up](uint64_t &x, uint64_t &y) {
+              if ((x > y) == up) {
+                const uint64_t z = x;
+                x = y;
+                y = z;
+              }
+            };
+            order(a0, a2);
+            order(a1, a3);
+            order(a0, a1);
+            order(a2, a3);
+            buf[i] = a0;
+            buf[i + h] = a1;
+            buf[i + stride] = a2;
+            buf[i + stride + h] = a3;
           }
+          stride >>= 2;
+        } else {
+          for (uint32_t q = tid; q < kpad / 2u; q += kSelThreads) {
+            const uint32_t i = 2u * q;
+            const uint64_t a = buf[i], b = buf[i + 1u];
+            if ((a > b) == ((i & size) == 0u)) {
+              buf[i] = b;
+              buf[i + 1u] = a;
+            }
+          }
+          stride = 0u;
         }
-        stride = 0u;
       }
     }
   }
   __syncthreads();
-  for (uint32_t i = tid; i < limit; i += kSelThreads) out[i] = buf[i];
+  const auto sorted_at = [&](uint32_t i) { return i < held ? sorted[i] : ~0ull; };
+  for (uint32_t i = tid; i < limit; i += kSelThreads)
+    __hip_atomic_store(&out[i], sorted_at(i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (tid < kSegs && !victims) st->seg[tid * 16u] = 0u;
+  if (tid == 0u && !victims)
+    __hip_atomic_store(&counters[kCntCandidates], n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  // the list finished last sees the other's keys and pairs both
+  __threadfence();
+  __syncthreads();
+  if (tid == 0u) s_cnt = atomicAdd(&st->done, 1u);
+  __syncthreads();
+  if (s_cnt == 0u) return;  // uniform
+  __threadfence();
+  if (tid == 0u) {
+    st->done = 0u;
+    s_fill = limit;  // the pairs that qualify: up to the first that does not
+    s_below = 0u;    // evicted
+  }
+  __syncthreads();
+  const uint64_t *other = victims ? cand_out : vict_out;
+  const auto pair_at = [&](uint32_t i, uint64_t &ck, uint64_t &vk) {
+    const uint64_t o = __hip_atomic_load(&other[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    ck = victims ? o : sorted_at(i);
+    vk = victims ? sorted_at(i) : o;
+  };
+  for (uint32_t i = tid; i < limit; i += kSelThreads) {
+    uint64_t ck, vk;
+    pair_at(i, ck, vk);
+    if (!pair_qualifies(ck, vk)) atomicMin(&s_fill, i);
+  }
+  __syncthreads();
+  const uint32_t loads = s_fill, stamp = counters[kCntStamp] + 1u;
+  for (uint32_t i = tid; i < loads; i += kSelThreads) {
+    uint64_t ck, vk;
+    pair_at(i, ck, vk);
+    if (apply_pair(tab, i, ck, vk, stamp)) atomicAdd(&s_below, 1u);
+  }
+  __syncthreads();
+  if (tid == 0u) {
+    counters[kCntLoads] = loads;
+    counters[kCntEvicted] = s_below;
+    counters[kCntStamp] = stamp;
+  }
 }
 
-// Candidate i takes victim i when the victim is free or strictly less
-// important.  Candidates descend and victims ascend in importance, so the
-// pairs that qualify are a prefix; its length is the first failure.
+// The pairing after the full sorts.
 __global__ void __launch_bounds__(256) pool_pair_kernel(const uint64_t *cand, const uint64_t *vict,
                                                         uint32_t limit, uint32_t *counters) {
   const uint32_t i = (uint32_t)(block_id() * 256u + threadIdx.x);
-  if (i >= limit) return;
-  const uint64_t ck = cand[i], vk = vict[i];
-  bool ok = ck != ~0ull;
-  if (ok && (uint32_t)(vk >> 32) != 0u) {
-    const float ci = __uint_as_float(~(uint32_t)(ck >> 32));
-    const float vi = __uint_as_float((uint32_t)(vk >> 32));
-    ok = vi < ci;
-  }
-  if (!ok) atomicMin(&counters[kCntLoads], i);
+  if (i < limit && !pair_qualifies(cand[i], vict[i])) atomicMin(&counters[kCntLoads], i);
 }
 
-// Applies the pairs: the victim's chunk leaves the lookup table, the
-// candidate takes its slot, and the load list for the mesher is written.
-// Old chunks (resident) and new ones (not resident) are disjoint sets and
-// every pair has its own slot, so the writes never collide.
 __global__ void __launch_bounds__(256) pool_apply_kernel(const uint64_t *cand, const uint64_t *vict,
-                                                         uint32_t limit, int32_t nc,
-                                                         uint32_t *lookup, uint32_t *slot_chunk,
-                                                         uint32_t *slot_stamp, int32_t *load_xyz,
-                                                         uint32_t *load_slot, uint32_t *counters) {
+                                                         uint32_t limit, PoolTables tab,
+                                                         uint32_t *counters) {
   const uint32_t i = (uint32_t)(block_id() * 256u + threadIdx.x);
   if (i >= limit || i >= counters[kCntLoads]) return;
-  const uint32_t sl = (uint32_t)vict[i], c = (uint32_t)cand[i];
-  const uint32_t old = slot_chunk[sl];
-  if (old != kNoSlot) {
-    lookup[old] = kNoSlot;
-    atomicAdd(&counters[kCntEvicted], 1u);
-  }
-  lookup[c] = sl;
-  slot_chunk[sl] = c;
-  slot_stamp[sl] = counters[kCntStamp];
-  const uint32_t n = (uint32_t)nc;
-  load_xyz[3 * i] = (int32_t)(c % n);
-  load_xyz[3 * i + 1] = (int32_t)((c / n) % n);
-  load_xyz[3 * i + 2] = (int32_t)(c / (n * n));
-  load_slot[i] = sl;
+  if (apply_pair(tab, i, cand[i], vict[i], counters[kCntStamp])) atomicAdd(&counters[kCntEvicted], 1u);
 }
 
 __global__ void pool_remesh_begin_kernel(uint32_t *counters) { counters[kCntRemesh] = 0u; }
@@ -508,6 +712,7 @@ struct meso_chunk_pool {
   uint64_t *cand = nullptr, *cand_sorted = nullptr, *vict = nullptr, *vict_sorted = nullptr;
   int32_t *load_xyz = nullptr, *remesh_xyz = nullptr;
   uint32_t *load_slot = nullptr, *remesh_slot = nullptr;
+  SelectState *select = nullptr;
   void *sort_tmp = nullptr;
   size_t sort_bytes = 0;
   uint64_t bytes = 0;
@@ -540,10 +745,16 @@ static void bake_directions(int32_t n, std::vector<float> &dirs) {
   }
 }
 
+// places of a candidate segment: the offsets of every kSegs-th workgroup
+static uint32_t seg_capacity(uint64_t cube) {
+  const uint64_t blocks = (cube + kKeyThreads - 1) / kKeyThreads;
+  return (uint32_t)((blocks + kSegs - 1) / kSegs * kKeyThreads);
+}
+
 static void pool_free(meso_chunk_pool *p) {
   void *ptrs[] = {p->lookup, p->slot_chunk, p->slot_stamp, p->slot_count, p->quads, p->counters,
                   p->cand, p->cand_sorted, p->vict, p->vict_sorted, p->load_xyz,
-                  p->remesh_xyz, p->load_slot, p->remesh_slot, p->sort_tmp};
+                  p->remesh_xyz, p->load_slot, p->remesh_slot, p->sort_tmp, p->select};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   delete p;
@@ -626,7 +837,7 @@ meso_status meso_chunk_pool_create(meso_context *ctx, meso_scene *scene, const m
   POOL_ALLOC(slot_count, cap * 4);
   POOL_ALLOC(quads, cap * (uint64_t)d.quads_per_slot * 4);
   POOL_ALLOC(counters, kCntWords * 4);
-  POOL_ALLOC(cand, p->cube * 8);
+  POOL_ALLOC(cand, (uint64_t)seg_capacity(p->cube) * kSegs * 8);  // at least one per offset
   POOL_ALLOC(cand_sorted, p->cube * 8);
   POOL_ALLOC(vict, cap * 8);
   POOL_ALLOC(vict_sorted, cap * 8);
@@ -634,6 +845,7 @@ meso_status meso_chunk_pool_create(meso_context *ctx, meso_scene *scene, const m
   POOL_ALLOC(load_slot, (uint64_t)d.max_loads * 4);
   POOL_ALLOC(remesh_xyz, cap * 12);
   POOL_ALLOC(remesh_slot, cap * 4);
+  POOL_ALLOC(select, sizeof(SelectState));
 #undef POOL_ALLOC
   if (st != MESO_OK) {
     pool_free(p);
@@ -658,6 +870,7 @@ meso_status meso_chunk_pool_create(meso_context *ctx, meso_scene *scene, const m
       hipMemsetAsync(p->slot_stamp, 0, cap * 4, ctx->stream) != hipSuccess ||
       hipMemsetAsync(p->slot_count, 0, cap * 4, ctx->stream) != hipSuccess ||
       hipMemsetAsync(p->counters, 0, kCntWords * 4, ctx->stream) != hipSuccess ||
+      hipMemsetAsync(p->select, 0, sizeof(SelectState), ctx->stream) != hipSuccess ||
       hipStreamSynchronize(ctx->stream) != hipSuccess) {
     (void)hipGetLastError();
     pool_free(p);
@@ -712,52 +925,53 @@ meso_status meso_chunk_pool_update(meso_chunk_pool *pool, const int32_t camera_c
   }
   const hipStream_t s = stream_of(pool->ctx, stream);
   const PoolGeom &g = pool->geom;
-  const int32_t cx = camera_chunk[0], cy = camera_chunk[1], cz = camera_chunk[2];
-  hipLaunchKernelGGL(pool_begin_kernel, dim3(1), dim3(1), 0, s, pool->counters, pool->limit);
-  MESO_HIP(hipGetLastError());
   const DevScene ds = pool->scene->dev();
+  const PoolView3 v{{camera_chunk[0], camera_chunk[1], camera_chunk[2]}, {f0, f1, f2}};
+  const bool map = pool->scene->kind == MESO_SCENE_BRICKMAP_U16;
+  const uint32_t cube = (uint32_t)pool->cube, cap = (uint32_t)g.capacity;
+  const PoolTables tab{g.nc, pool->lookup, pool->slot_chunk, pool->slot_stamp, pool->load_xyz,
+                       pool->load_slot};
   // limits up to kSelMax select the first keys of lists up to kSelListMax
   // keys (candidates: at most one per cube offset; victims: one per slot);
   // larger limits or longer lists sort the lists
-  const bool select = pool->limit <= kSelMax && (uint64_t)pool->cube <= kSelListMax &&
-                      (uint64_t)pool->geom.capacity <= kSelListMax;
-  if (pool->scene->kind == MESO_SCENE_BRICKMAP_U16)
-    hipLaunchKernelGGL(pool_rank_kernel<2>, grid_1d((pool->cube + 255) / 256), dim3(256), 0, s,
-                       ds, g, cx, cy, cz, f0, f1, f2, pool->lookup, pool->cand, pool->cube,
-                       pool->counters, select);
-  else
-    hipLaunchKernelGGL(pool_rank_kernel<3>, grid_1d((pool->cube + 255) / 256), dim3(256), 0, s,
-                       ds, g, cx, cy, cz, f0, f1, f2, pool->lookup, pool->cand, pool->cube,
-                       pool->counters, select);
-  MESO_HIP(hipGetLastError());
-  const uint64_t cap = (uint64_t)g.capacity;
-  hipLaunchKernelGGL(pool_victim_kernel, grid_1d((cap + 255) / 256), dim3(256), 0, s, g, cx, cy,
-                     cz, f0, f1, f2, pool->slot_chunk, pool->vict);
-  MESO_HIP(hipGetLastError());
-  if (select) {
+  if (pool->limit <= kSelMax && cube <= kSelListMax && cap <= kSelListMax) {
+    const uint32_t rank_blocks = (cube + kKeyThreads - 1u) / kKeyThreads,
+                   vict_blocks = (cap + kKeyThreads - 1u) / kKeyThreads;
+    const auto keys = map ? pool_keys_kernel<2> : pool_keys_kernel<3>;
+    hipLaunchKernelGGL(keys, dim3(rank_blocks + vict_blocks), dim3(kKeyThreads), 0, s, ds, g, v,
+                       pool->lookup, pool->slot_chunk, cube, rank_blocks, seg_capacity(pool->cube),
+                       pool->cand, pool->vict, pool->select);
+    MESO_HIP(hipGetLastError());
     uint32_t kpad = 1u;
     while (kpad < pool->limit) kpad <<= 1;
     hipLaunchKernelGGL(pool_select_kernel, dim3(2), dim3(kSelThreads), 0, s, pool->cand,
-                       pool->vict, (uint32_t)cap, pool->limit, kpad, pool->counters,
-                       pool->cand_sorted, pool->vict_sorted);
+                       pool->vict, cap, seg_capacity(pool->cube), pool->limit, kpad, pool->select,
+                       pool->cand_sorted, pool->vict_sorted, tab, pool->counters);
     MESO_HIP(hipGetLastError());
   } else {
+    hipLaunchKernelGGL(pool_begin_kernel, dim3(1), dim3(1), 0, s, pool->counters, pool->limit);
+    MESO_HIP(hipGetLastError());
+    const auto rank = map ? pool_rank_kernel<2> : pool_rank_kernel<3>;
+    hipLaunchKernelGGL(rank, dim3((cube + 255u) / 256u), dim3(256), 0, s, ds, g, v, pool->lookup,
+                       pool->cand, cube, pool->counters);
+    MESO_HIP(hipGetLastError());
+    hipLaunchKernelGGL(pool_victim_kernel, dim3((cap + 255u) / 256u), dim3(256), 0, s, g, v,
+                       pool->slot_chunk, pool->vict);
+    MESO_HIP(hipGetLastError());
     size_t b = pool->sort_bytes;
     MESO_HIP(rocprim::radix_sort_keys(pool->sort_tmp, b, pool->cand, pool->cand_sorted,
                                       (size_t)pool->cube, 0, 64, s));
     b = pool->sort_bytes;
     MESO_HIP(rocprim::radix_sort_keys(pool->sort_tmp, b, pool->vict, pool->vict_sorted,
                                       (size_t)cap, 0, 64, s));
+    const dim3 grid = grid_1d(((uint64_t)pool->limit + 255) / 256);
+    hipLaunchKernelGGL(pool_pair_kernel, grid, dim3(256), 0, s, pool->cand_sorted,
+                       pool->vict_sorted, pool->limit, pool->counters);
+    MESO_HIP(hipGetLastError());
+    hipLaunchKernelGGL(pool_apply_kernel, grid, dim3(256), 0, s, pool->cand_sorted,
+                       pool->vict_sorted, pool->limit, tab, pool->counters);
+    MESO_HIP(hipGetLastError());
   }
-  const uint64_t lim = pool->limit;
-  hipLaunchKernelGGL(pool_pair_kernel, grid_1d((lim + 255) / 256), dim3(256), 0, s,
-                     pool->cand_sorted, pool->vict_sorted, pool->limit, pool->counters);
-  MESO_HIP(hipGetLastError());
-  hipLaunchKernelGGL(pool_apply_kernel, grid_1d((lim + 255) / 256), dim3(256), 0, s,
-                     pool->cand_sorted, pool->vict_sorted, pool->limit, g.nc, pool->lookup,
-                     pool->slot_chunk, pool->slot_stamp, pool->load_xyz, pool->load_slot,
-                     pool->counters);
-  MESO_HIP(hipGetLastError());
   return launch_mesh_slotted(pool->ctx, pool->scene, pool->load_xyz, pool->load_slot,
                              pool->counters + kCntLoads, (int32_t)pool->limit,
                              pool->desc.mesh_mode, pool->slot_count, pool->quads,
