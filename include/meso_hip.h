@@ -588,6 +588,9 @@ meso_status meso_serve_wait(meso_server *srv, uint64_t ticket, int64_t timeout_u
                             double *latency_us);
 /* Copy a completed result to host memory and release its HBM budget. */
 meso_status meso_serve_take(meso_server *srv, uint64_t ticket, const meso_host_outputs *dst);
+/* The same, with hit_index an array of 64-bit indices whatever the result
+ * holds (index_bytes still says what that is, or 0). */
+meso_status meso_serve_take_wide(meso_server *srv, uint64_t ticket, const meso_host_outputs *dst);
 meso_status meso_serve_stats_get(meso_server *srv, meso_serve_stats *out);
 meso_status meso_serve_stop(meso_server *srv);
 

@@ -186,6 +186,7 @@ _SIGS = {
     "meso_serve_poll": (C.c_int32, [P, C.c_uint64, C.POINTER(C.c_int32)]),
     "meso_serve_wait": (C.c_int32, [P, C.c_uint64, C.c_int64, C.POINTER(C.c_double)]),
     "meso_serve_take": (C.c_int32, [P, C.c_uint64, P]),
+    "meso_serve_take_wide": (C.c_int32, [P, C.c_uint64, P]),
     "meso_serve_stats_get": (C.c_int32, [P, P]),
     "meso_serve_stop": (C.c_int32, [P]),
     "meso_chunk_pool_create": (C.c_int32, [P, P, P, PP]),
