@@ -790,10 +790,15 @@ __device__ __forceinline__ uint32_t hash32(uint32_t x) {
 // counter-based hashes, lifted by z = sqrt(1 - r^2).
 __device__ __forceinline__ void ao_direction(uint32_t seed, uint32_t pixel, uint32_t sample,
                                              int face, float dir[3]) {
-  float a = 0.0f, b = 0.0f, r2 = 0.0f;
+  float a, b, r2;
   const uint32_t base = hash32(hash32(seed) ^ pixel);
-  bool ok = false;
-  for (uint32_t k = 0; k < 16u; k++) {
+  uint32_t k = 0;
+  // one try a trip: the compiler made four at a time of the loop, with eight
+  // quarter-rate multiplies, which cost more than the 3.6 trips that the
+  // unluckiest lane of a wave needs on average (3840x2160 caves with four AO
+  // rays 1672 us, now 1635)
+#pragma clang loop vectorize(disable) interleave(disable) unroll(disable)
+  do {
     uint32_t h = hash32(base ^ (sample * 16u + k));
     a = (float)(h & 0xFFFFu) * (1.0f / 32768.0f);
     a = a - 1.0f;
@@ -801,12 +806,9 @@ __device__ __forceinline__ void ao_direction(uint32_t seed, uint32_t pixel, uint
     b = b - 1.0f;
     float aa = a * a, bb = b * b;
     r2 = aa + bb;
-    if (r2 < 1.0f) {
-      ok = true;
-      break;
-    }
-  }
-  if (!ok) {
+    k++;
+  } while (r2 >= 1.0f && k < 16u);
+  if (r2 >= 1.0f) {
     a = 0.0f;
     b = 0.0f;
     r2 = 0.0f;
