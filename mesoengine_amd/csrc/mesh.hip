@@ -726,15 +726,20 @@ __global__ void __launch_bounds__(T) mesh_batched_kernel(
       build_masks<ES, T>(L, SceneRows<SRC>{ss.s, cx * 32, cy * 32, cz * 32});
     }
     const uint32_t chunk_total = chunk_count<GREEDY, T>(L);
-    if (t == 0) {
-      // publish the aggregate, then add up predecessors until an inclusive one.
+    if (t < 64) {  // one wave: publish, then add up the chunks before this one
       // The value travels inside the status word and no other data is
       // exchanged, so the status accesses are relaxed: agent-scope release /
       // acquire would write back and invalidate this XCD's whole L2 at every
       // chunk (and every spin), evicting the chunk data of the other
       // workgroups on it.
-      __hip_atomic_store(&work->status[c], kAgg | (uint64_t)chunk_total, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
+      if (t == 0)
+        __hip_atomic_store(&work->status[c], kAgg | (uint64_t)chunk_total, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      // 64 predecessors a look, the nearest in lane 0: a status is read at the
+      // memory side, most of a microsecond, and chunks that started together
+      // have as many between them and the last one with its sum (read one by
+      // one: 4096 greedy chunks 230 us, now 212; 1331 culled ones 95, now 89;
+      // 2,621 chunks of a scene 145, now 131).
       uint64_t before = 0;
       int64_t j = (int64_t)c - 1;
       uint32_t spins = 0;
@@ -745,30 +750,40 @@ __global__ void __launch_bounds__(T) mesh_batched_kernel(
         // wave exits.  The chunk's outputs are then wrong and the error word
         // says so (meso_mesh_check).
         if (spins >= spin_limit) {
-          atomicOr(&work->error, 1u);
+          if (t == 0) atomicOr(&work->error, 1u);
           break;
         }
-        const uint64_t st = __hip_atomic_load(&work->status[j], __ATOMIC_RELAXED,
-                                              __HIP_MEMORY_SCOPE_AGENT);
-        if (st & kInc) {
-          before += st & kValMask;
-          break;
+        const int64_t k = j - t;
+        const uint64_t st = k < 0 ? kInc
+                                  : __hip_atomic_load(&work->status[k], __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t inc = __ballot((st & kInc) != 0), none = __ballot((st & (kInc | kAgg)) == 0);
+        // the lanes before the first one that has published nothing, and of
+        // these up to the first that holds the sum of all before it
+        const int n_ready = none ? __builtin_ctzll(none) : 64;
+        const int at_inc = inc ? __builtin_ctzll(inc) : 64;
+        const bool done = at_inc < n_ready;
+        const int n_take = done ? at_inc + 1 : n_ready;
+        uint64_t v = t < n_take ? st & kValMask : 0;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+        before += v;
+        if (done) break;
+        j -= n_take;
+        if (n_take == 0) {
+          spins++;
+          __builtin_amdgcn_s_sleep(1);
         }
-        if (st & kAgg) {
-          before += st & kValMask;
-          j--;
-          continue;
-        }
-        spins++;
-        __builtin_amdgcn_s_sleep(1);
       }
-      __hip_atomic_store(&work->status[c], kInc | (before + chunk_total), __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_AGENT);
-      counts[c] = chunk_total;
-      prefix[c] = (uint32_t)before;
-      if (c == n_chunks - 1) *total = before + chunk_total;
-      L.base_lo = (uint32_t)before;
-      L.base_hi = (uint32_t)(before >> 32);
+      if (t == 0) {
+        __hip_atomic_store(&work->status[c], kInc | (before + chunk_total), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+        counts[c] = chunk_total;
+        prefix[c] = (uint32_t)before;
+        if (c == n_chunks - 1) *total = before + chunk_total;
+        L.base_lo = (uint32_t)before;
+        L.base_hi = (uint32_t)(before >> 32);
+      }
     }
     __syncthreads();
     const uint64_t base = ((uint64_t)L.base_hi << 32) | L.base_lo;
