@@ -26,6 +26,7 @@
 //     its output offset by an ordered decoupled look-back over the chunks
 //     ticketed before it, so one persistent launch writes one compact quad
 //     buffer plus per-chunk counts and exclusive prefixes.
+#include <algorithm>
 #include <cstddef>
 #include <type_traits>
 
@@ -513,9 +514,10 @@ __device__ __forceinline__ int plane_of(const MeshLds &L, uint32_t q) {
 constexpr uint32_t kRun = 8;
 
 template <int T>
-__device__ __forceinline__ void culled_emit_balanced(const MeshLds &L, uint32_t total,
-                                                     uint32_t *out, uint64_t base, uint64_t cap) {
-  for (uint32_t q0 = threadIdx.x * kRun; q0 < total; q0 += (uint32_t)T * kRun) {
+__device__ __forceinline__ void culled_emit_balanced(const MeshLds &L, uint32_t first,
+                                                     uint32_t total, uint32_t *out, uint64_t base,
+                                                     uint64_t cap) {
+  for (uint32_t q0 = first + threadIdx.x * kRun; q0 < total; q0 += (uint32_t)T * kRun) {
     const uint32_t q1 = q0 + kRun < total ? q0 + kRun : total;
     int pl = plane_of(L, q0);
     PlaneView p = plane_view(pl >> 5, pl & 31);
@@ -571,12 +573,12 @@ constexpr uint32_t kMarks = 4096u, kMarkStep = kMarks - 64u;
 static_assert(kEy + kMarks / 2u <= kEyT, "the marks lie over Ey, Ez and OT");
 
 template <int T>
-__device__ __forceinline__ void greedy_emit(GreedyLds &L, uint32_t total, uint32_t *out,
-                                            uint64_t base, uint64_t cap) {
+__device__ __forceinline__ void greedy_emit(GreedyLds &L, uint32_t first, uint32_t total,
+                                            uint32_t *out, uint64_t base, uint64_t cap) {
   const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
   uint16_t *marks = (uint16_t *)(L.M + kEy);  // marks[64 + q - w0]
   uint32_t *marks2 = L.M + kEy;
-  for (uint32_t w0 = 0; w0 < total; w0 += kMarkStep) {  // uniform
+  for (uint32_t w0 = first; w0 < total; w0 += kMarkStep) {  // uniform
     for (uint32_t k = t; k < kMarks / 2u; k += (uint32_t)T) marks2[k] = 0u;
     __syncthreads();
     if (t < (uint32_t)kPlanes) {
@@ -674,16 +676,27 @@ __device__ __forceinline__ uint32_t chunk_count(LdsOf<GREEDY> &L) {
   return total;
 }
 
-// The counted chunk's quads at out[base ...], up to out[cap]; every thread of
-// the workgroup calls it after a barrier.
+// Part `part` of `parts` of the counted chunk's quads at out[base ...], up to
+// out[cap]; every thread of the workgroup calls it after a barrier.
 template <bool GREEDY, int T>
-__device__ __forceinline__ void chunk_emit(LdsOf<GREEDY> &L, uint32_t total, uint32_t *out,
-                                           uint64_t base, uint64_t cap) {
+__device__ __forceinline__ void chunk_emit(LdsOf<GREEDY> &L, uint32_t total, uint32_t part,
+                                           uint32_t parts, uint32_t *out, uint64_t base,
+                                           uint64_t cap) {
+  const uint32_t first = total * part / parts, end = total * (part + 1u) / parts;
   if constexpr (GREEDY)
-    greedy_emit<T>(L, total, out, base, cap);
+    greedy_emit<T>(L, first, end, out, base, cap);
   else
-    culled_emit_balanced<T>(L, total, out, base, cap);
+    culled_emit_balanced<T>(L, first, end, out, base, cap);
 }
+
+// Workgroups per chunk of a voxel array where there are fewer chunks than CUs:
+// each builds the chunk's masks and counts it (7.5 us), and writes its part of
+// the quads, of which such chunks may have many: one chunk of 12,516 greedy
+// quads takes 32.5 us with one workgroup, 21.2 with two, 15.1 with four and
+// 14.0 with eight; 8 in a batch 24.3 and 19.2, 100 (two each) 25.9 and 22.1.
+// Chunks of a scene hold a surface, some hundred quads, and gain nothing (40 of
+// them with their edit 27.1 us either way).
+constexpr uint32_t kMaxParts = 4;
 
 // look-back status word: flag in bits 62-63 (1 = aggregate, 2 = inclusive)
 constexpr uint64_t kAgg = 1ull << 62, kInc = 2ull << 62, kValMask = (1ull << 62) - 1;
@@ -707,14 +720,18 @@ struct SceneSource {
 template <int ES, bool GREEDY, int SRC, int T>
 __global__ void __launch_bounds__(T) mesh_batched_kernel(
     meso_chunk_source src, SceneSource ss, uint32_t *counts, uint32_t *prefix, uint32_t *quads,
-    uint64_t capacity, unsigned long long *total, MeshWork *work, uint32_t spin_limit) {
+    uint64_t capacity, unsigned long long *total, MeshWork *work, uint32_t spin_limit,
+    uint32_t parts) {
+  constexpr bool kSplit = SRC == 0 && T == kChunkBlock;  // see kMaxParts
   __shared__ LdsOf<GREEDY> L;
   const int t = (int)threadIdx.x;
   const uint32_t n_chunks = (uint32_t)(SRC == 0 ? src.n_chunks : ss.n_chunks);
   for (;;) {
     if (t == 0) L.chunk = atomicAdd(&work->ticket, 1u);
     __syncthreads();
-    const uint32_t c = L.chunk;
+    const uint32_t ticket = L.chunk;
+    const uint32_t c = kSplit ? ticket / parts : ticket;
+    const uint32_t part = kSplit ? ticket - c * parts : 0u;
     if (c >= n_chunks) break;  // uniform: every wave leaves
     if constexpr (SRC == 0) {
       build_masks<ES, T>(L, chunk_addr(src, c));
@@ -732,7 +749,7 @@ __global__ void __launch_bounds__(T) mesh_batched_kernel(
       // acquire would write back and invalidate this XCD's whole L2 at every
       // chunk (and every spin), evicting the chunk data of the other
       // workgroups on it.
-      if (t == 0)
+      if (t == 0 && part == 0)
         __hip_atomic_store(&work->status[c], kAgg | (uint64_t)chunk_total, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_AGENT);
       // 64 predecessors a look, the nearest in lane 0: a status is read at the
@@ -744,11 +761,11 @@ __global__ void __launch_bounds__(T) mesh_batched_kernel(
       int64_t j = (int64_t)c - 1;
       uint32_t spins = 0;
       while (j >= 0) {
-        // chunk j was ticketed earlier, so its workgroup is resident and will
-        // publish; the bound (the context's spin limit, 2^24 polls unless the
-        // host lowers it to inject the failure) only guarantees that every
-        // wave exits.  The chunk's outputs are then wrong and the error word
-        // says so (meso_mesh_check).
+        // chunk j's first part was ticketed earlier, so its workgroup is
+        // resident and will publish; the bound (the context's spin limit, 2^24
+        // polls unless the host lowers it to inject the failure) only
+        // guarantees that every wave exits.  The chunk's outputs are then
+        // wrong and the error word says so (meso_mesh_check).
         if (spins >= spin_limit) {
           if (t == 0) atomicOr(&work->error, 1u);
           break;
@@ -776,18 +793,20 @@ __global__ void __launch_bounds__(T) mesh_batched_kernel(
         }
       }
       if (t == 0) {
-        __hip_atomic_store(&work->status[c], kInc | (before + chunk_total), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-        counts[c] = chunk_total;
-        prefix[c] = (uint32_t)before;
-        if (c == n_chunks - 1) *total = before + chunk_total;
+        if (part == 0) {
+          __hip_atomic_store(&work->status[c], kInc | (before + chunk_total), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+          counts[c] = chunk_total;
+          prefix[c] = (uint32_t)before;
+          if (c == n_chunks - 1) *total = before + chunk_total;
+        }
         L.base_lo = (uint32_t)before;
         L.base_hi = (uint32_t)(before >> 32);
       }
     }
     __syncthreads();
     const uint64_t base = ((uint64_t)L.base_hi << 32) | L.base_lo;
-    chunk_emit<GREEDY, T>(L, chunk_total, quads, base, capacity);
+    chunk_emit<GREEDY, T>(L, chunk_total, part, kSplit ? parts : 1u, quads, base, capacity);
     __syncthreads();
   }
 }
@@ -819,7 +838,7 @@ __global__ void __launch_bounds__(T) mesh_slotted_kernel(
     const uint64_t base = (uint64_t)slot * per_slot;
     if (t == 0) slot_count[slot] = chunk_total;
     __syncthreads();
-    chunk_emit<GREEDY, T>(L, chunk_total, quads, base, base + per_slot);
+    chunk_emit<GREEDY, T>(L, chunk_total, 0, 1, quads, base, base + per_slot);
     if (!tickets) break;
     if (t == 0) L.chunk = atomicAdd(&ticket[0], 1u);
     __syncthreads();
@@ -839,9 +858,9 @@ __global__ void __launch_bounds__(T) mesh_plain_kernel(const void *voxels, uint3
   const ChunkAddr a{voxels, 0, 32, 1024};
   build_masks<ES, T>(L, a);
   const uint32_t chunk_total = chunk_count<GREEDY, T>(L);
-  if (threadIdx.x == 0) *count = chunk_total;
+  if (threadIdx.x == 0 && blockIdx.x == 0) *count = chunk_total;
   __syncthreads();
-  chunk_emit<GREEDY, T>(L, chunk_total, quads, 0, capacity);
+  chunk_emit<GREEDY, T>(L, chunk_total, blockIdx.x, gridDim.x, quads, 0, capacity);
 }
 
 template <int ES, bool GREEDY, int SRC, int T>
@@ -858,13 +877,16 @@ static meso_status launch_batched_w(meso_context *ctx, const meso_chunk_source &
     if (per_cu < 1) per_cu = 1;
     grid = per_cu * ctx->props.multiProcessorCount;
   }
-  if (grid > n_chunks) grid = n_chunks;
+  const int parts = SRC == 0 && T == kChunkBlock
+                        ? std::clamp(ctx->props.multiProcessorCount / n_chunks, 1, (int)kMaxParts)
+                        : 1;
+  if (grid > n_chunks * parts) grid = n_chunks * parts;
   meso_status st = launch_zero(d_work, meso_mesh_workspace_bytes(n_chunks), stream);
   if (st != MESO_OK) return st;
   hipLaunchKernelGGL((mesh_batched_kernel<ES, GREEDY, SRC, T>), dim3(grid), dim3(T), 0,
                      stream, src, ss, d_counts, d_prefix, d_quads, capacity,
                      (unsigned long long *)d_total, (MeshWork *)d_work,
-                     ctx->lookback_spin_limit);
+                     ctx->lookback_spin_limit, (uint32_t)parts);
   MESO_HIP(hipGetLastError());
   return MESO_OK;
 }
@@ -1010,8 +1032,8 @@ meso_status launch_mesh_slotted(meso_context *ctx, const meso_scene *scene, cons
 template <int ES, bool GREEDY>
 static void launch_plain_t(const void *voxels, uint32_t *d_count, uint32_t *d_quads,
                            uint32_t capacity, hipStream_t stream) {
-  hipLaunchKernelGGL((mesh_plain_kernel<ES, GREEDY, kChunkBlock>), dim3(1), dim3(kChunkBlock), 0, stream, voxels,
-                     d_count, d_quads, capacity);
+  hipLaunchKernelGGL((mesh_plain_kernel<ES, GREEDY, kChunkBlock>), dim3(kMaxParts), dim3(kChunkBlock), 0,
+                     stream, voxels, d_count, d_quads, capacity);
 }
 
 meso_status launch_mesh_plain(const void *voxels, int32_t es, uint32_t mode, uint32_t *d_count,
