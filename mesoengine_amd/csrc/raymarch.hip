@@ -121,7 +121,7 @@ __device__ __forceinline__ bool walk_part(const DevScene &s, const Ray &r, WalkS
     tmax = to < tmax ? to : tmax;
   }
   if (part > 0u) dense_skip(r, w, from);
-  return walk_dense(s, r, e, w, tmax, material);
+  return walk_dense<kDenseAhead>(s, r, e, w, tmax, material);
 }
 
 __global__ void __launch_bounds__(64) raymarch_dense_small_kernel(DevScene s, DevCamera cam,

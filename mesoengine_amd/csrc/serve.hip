@@ -439,7 +439,7 @@ __global__ void __launch_bounds__(kServeThreads)
       const int32_t py = (int32_t)((u / packets_x) * kServePacket + (lane >> 3));
       if (px < cam.width && py < cam.height) {
         switch (kind) {
-          case MESO_SCENE_DENSE_U8: serve_pixel<1>(d, scene, cam, px, py); break;
+          case MESO_SCENE_DENSE_U8: serve_pixel<kDenseShort>(d, scene, cam, px, py); break;
           case MESO_SCENE_BRICKMAP_U16: serve_pixel<2>(d, scene, cam, px, py); break;
           default: serve_pixel<3>(d, scene, cam, px, py); break;
         }
@@ -711,8 +711,17 @@ class ResultReader {
 
   // parts in the order they lie in the block; those without dst are skipped.
   hipError_t read(const uint8_t *block, const ResultPart *parts, int n) {
+    uint64_t total = 0;
+    int wanted = 0;
+    for (int k = 0; k < n; k++) {
+      total += parts[k].dst ? parts[k].bytes : 0;
+      wanted += parts[k].dst ? 1 : 0;
+    }
+    // one array of one chunk has nothing to overlap: 200 queued requests whose
+    // faces alone are taken ran 13.2 ms with a plain copy and 14.6 staged
+    if (!ready_ || (wanted < 2 && total <= kChunkBytes)) return read_direct(block, parts, n);
     std::unique_lock<std::mutex> one(take_mu_, std::try_to_lock);
-    if (!ready_ || !one.owns_lock()) return read_direct(block, parts, n);
+    if (!one.owns_lock()) return read_direct(block, parts, n);
     return read_staged(block, parts, n);
   }
 

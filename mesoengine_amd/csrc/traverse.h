@@ -251,6 +251,10 @@ struct WalkCache {
   }
 };
 
+// KIND of a dense grid walked a few cells at a time, for a kernel of all scene
+// kinds that has no registers for more
+constexpr int kDenseShort = 4;
+
 enum : int { kWalkOn = 0, kWalkHit = 1, kWalkOut = 2 };
 
 // One step of a walk from a cell whose entry t is below tmax: kWalkHit when
@@ -270,7 +274,7 @@ __device__ __forceinline__ int walk_step(const DevScene &s, const Ray &r, WalkSt
                                          StepCounts &cnt) {
   const int32_t n = s.n;
   if (COUNT) cnt.n_iter++;
-  if constexpr (KIND == 1) {
+  if constexpr (KIND == 1 || KIND == kDenseShort) {
     if (COUNT) cnt.n_vox++;
     const uint8_t v = s.dense[lin3(w.cell[0], w.cell[1], w.cell[2], n)];
     if (v) {
@@ -351,7 +355,7 @@ __device__ __forceinline__ int walk_step(const DevScene &s, const Ray &r, WalkSt
 }
 
 // Dense grid: the cells a ray visits do not depend on what they hold, so a walk
-// finds its next kDenseAhead cells first and then loads them together.  One
+// finds its next AHEAD cells first and then loads them together.  One
 // voxel load at a time bounded it by latency: a 256x256 frame of a 256^3 grid
 // has one wave per SIMD, and each of some 200 steps waited for its load (148
 // us, now 53; 4 cells at a time 79, 8 70 and 16 68 before the steps below).
@@ -366,6 +370,11 @@ __device__ __forceinline__ int walk_step(const DevScene &s, const Ray &r, WalkSt
 // made exact, was 5 times slower, lanes in blocks and lanes in steps running
 // both ways in every trip.)
 constexpr int kDenseAhead = 16;
+// where registers are short: the serving kernel's 131 with 16 left 3 waves a
+// SIMD, 103 leave 4 (200 queued requests, none of them dense: 12,050 Mrays/s
+// with 16, 13,370 with 4 workgroups a CU, 12,880 with the 5 that fit with no
+// cells ahead, which contend for the claims)
+constexpr int kDenseAheadShort = 4;
 constexpr int32_t kDenseIndexed = 1625;  // 1625^3 < 2^32: 32-bit voxel indices
 
 struct DenseRay {
@@ -416,6 +425,7 @@ __device__ __forceinline__ float dense_step(const Ray &r, float plane[3], int &a
   return t;
 }
 
+template <int AHEAD>
 __device__ __forceinline__ bool walk_dense(const DevScene &s, const Ray &r, const DenseRay &e,
                                            WalkState &w, float tmax, uint16_t &material) {
   const uint32_t n = (uint32_t)s.n;
@@ -436,12 +446,12 @@ __device__ __forceinline__ bool walk_dense(const DevScene &s, const Ray &r, cons
   for (;;) {
     const float from[3] = {plane[0], plane[1], plane[2]};
     const uint32_t first = idx;
-    uint32_t at[kDenseAhead];
+    uint32_t at[AHEAD];
     bool on = true;
     float t = 0.0f;
     int ax = 0;
 #pragma unroll
-    for (int i = 0; i < kDenseAhead; i++) {
+    for (int i = 0; i < AHEAD; i++) {
       // cells past the walk's end are read as the batch's first cell, which is
       // its first solid one or empty
       at[i] = on ? idx : first;
@@ -450,11 +460,11 @@ __device__ __forceinline__ bool walk_dense(const DevScene &s, const Ray &r, cons
       on = on && t < t_lim;
     }
     uint32_t solid = 0;
-    uint8_t v[kDenseAhead];
+    uint8_t v[AHEAD];
 #pragma unroll
-    for (int i = 0; i < kDenseAhead; i++) v[i] = s.dense[at[i]];
+    for (int i = 0; i < AHEAD; i++) v[i] = s.dense[at[i]];
 #pragma unroll
-    for (int i = 0; i < kDenseAhead; i++) solid |= (v[i] ? 1u : 0u) << i;
+    for (int i = 0; i < AHEAD; i++) solid |= (v[i] ? 1u : 0u) << i;
     bool hit = solid != 0u;
     if (hit || !on) {
       // the batch's steps once more, to the first solid cell for its t, face
@@ -623,11 +633,12 @@ template <int KIND, bool COUNT>
 __device__ __forceinline__ bool walk(const DevScene &s, const Ray &r, WalkState &w, float tmax,
                                      uint16_t &material, StepCounts &cnt) {
   if (!(w.t < tmax)) return false;
-  if constexpr (KIND == 1 && !COUNT) {
+  if constexpr ((KIND == 1 || KIND == kDenseShort) && !COUNT) {
+    constexpr int ahead = KIND == 1 ? kDenseAhead : kDenseAheadShort;
     DenseRay e;
-    if (e.setup(s, r)) return walk_dense(s, r, e, w, tmax, material);
+    if (e.setup(s, r)) return walk_dense<ahead>(s, r, e, w, tmax, material);
   }
-  if constexpr (KIND != 1 && !COUNT) return walk_bricks<KIND>(s, r, w, tmax, material);
+  if constexpr ((KIND == 2 || KIND == 3) && !COUNT) return walk_bricks<KIND>(s, r, w, tmax, material);
   WalkCache c;
   c.reset();
   for (;;) {

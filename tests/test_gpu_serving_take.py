@@ -94,6 +94,15 @@ def test_wide_indices(ctx, setup):
     sc.destroy()
 
 
+@pytest.mark.parametrize("n", [5, 16, 61])
+def test_dense_scenes(ctx, setup, n):
+    _, srv = setup
+    sc = ctx.scene_generate(L.GEN_SPHERES, L.SCENE_DENSE_U8, n, 2, 5)
+    for size in [(1, 1), (123, 77), (640, 361)]:
+        _same(_served(srv, sc, *size), _plain(ctx, sc, *size))
+    sc.destroy()
+
+
 def test_threads_take_at_once(ctx, setup):
     sc, srv = setup
     sizes = [(1500, 901), (1201, 700), (64, 64)]
