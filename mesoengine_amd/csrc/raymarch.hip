@@ -1,7 +1,8 @@
 // Raymarch kernels: one lane per pixel, wave64 packets of 8x8 pixels so the
-// rays of a wave fetch the same bricks.  Tiled variants remap workgroups so
-// that each XCD (own L2) renders a contiguous band of tiles; the persistent
-// variant keeps every wave slot busy and pulls packets from per-band queues.
+// rays of a wave fetch the same bricks (small dense frames: four lanes per
+// pixel).  Tiled variants hand rows of tiles to the XCDs in turn; the
+// persistent variant keeps every wave slot busy and pulls packets from
+// per-band queues.
 #include "traverse.h"
 
 namespace meso {
