@@ -77,53 +77,10 @@ __global__ void __launch_bounds__(TW *TH) raymarch_kernel(DevScene s, DevCamera 
 // short, are dealt out instead, one sample in four to a lane.  The rays' set-up
 // is done four times.  256x256 pixels over 256^3 voxels with shadows, a long
 // view, 120 us, now 60; 318x318 over 77^3 with shadows and two AO rays 42 and 22.
-constexpr int kDenseParts = 4;
+//
 // The most 8x8 waves per SIMD of a frame that goes this way: 640x360, 3.5 a
 // SIMD, takes 75 us instead of 119, but 800x600, 7.3 a SIMD, 112 instead of 103.
 constexpr uint32_t kSmallWaves = 4;
-
-// The part's start on a ray that walk_dense() takes: the cell after every plane
-// with a t below `from` has been crossed, which is where the walk from w.cell
-// would be then.  A plane at t is within 2^-5 of the ray's point at t, so the
-// first plane with a t of at least `from` is one of four.
-__device__ __forceinline__ void dense_skip(const Ray &r, WalkState &w, float from) {
-#pragma unroll
-  for (int a = 0; a < 3; a++) {
-    if (r.step[a] == 0) continue;
-    const float s = (float)r.step[a], first = (float)(w.cell[a] + r.pos[a]);
-    const float dt = r.d[a] * from;
-    const float mid = __builtin_rintf(r.o[a] + dt);
-    float p = mid + 2.0f * s;
-#pragma unroll
-    for (int k = 1; k >= -1; k--) {
-      const float c = mid + (float)k * s;
-      p = plane_t(r.o[a], r.inv[a], c) >= from ? c : p;
-    }
-    p = (p - first) * s > 0.0f ? p : first;
-    w.cell[a] = (int32_t)p - r.pos[a];
-  }
-}
-
-// walk() by the four lanes of a pixel: true in those that hit.  A start cell
-// that is solid was the last cell of the part before, whose lane then has it.
-__device__ __forceinline__ bool walk_part(const DevScene &s, const Ray &r, WalkState &w, float tmax,
-                                          uint32_t part, uint16_t &material) {
-  if (!(w.t < tmax)) return false;
-  DenseRay e;
-  if (!e.setup(s, r)) {
-    StepCounts cnt;
-    return part == 0u && walk<1, false>(s, r, w, tmax, material, cnt);
-  }
-  const float t_lim = tmax < e.t_out ? tmax : e.t_out;
-  const float step = (t_lim - w.t) * (1.0f / kDenseParts);
-  const float from = w.t + step * (float)part;
-  if (part + 1u < (uint32_t)kDenseParts) {
-    const float to = w.t + step * (float)(part + 1u);
-    tmax = to < tmax ? to : tmax;
-  }
-  if (part > 0u) dense_skip(r, w, from);
-  return walk_dense<kDenseAhead>(s, r, e, w, tmax, material);
-}
 
 __global__ void __launch_bounds__(64) raymarch_dense_small_kernel(DevScene s, DevCamera cam,
                                                                   uint32_t flags, DevShading sh,

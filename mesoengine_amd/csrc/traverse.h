@@ -647,6 +647,70 @@ __device__ __forceinline__ bool walk(const DevScene &s, const Ray &r, WalkState 
   }
 }
 
+// A dense ray walked in parts of its stretch of t, one by each of kDenseParts lanes.
+constexpr int kDenseParts = 4;
+
+// The part's start on a ray that walk_dense() takes: the cell after every plane
+// with a t below `from` has been crossed, which is where the walk from w.cell
+// would be then.  A plane at t is within 2^-5 of the ray's point at t, so the
+// first plane with a t of at least `from` is one of four.
+__device__ __forceinline__ void dense_skip(const Ray &r, WalkState &w, float from) {
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    if (r.step[a] == 0) continue;
+    const float s = (float)r.step[a], first = (float)(w.cell[a] + r.pos[a]);
+    const float dt = r.d[a] * from;
+    const float mid = __builtin_rintf(r.o[a] + dt);
+    float p = mid + 2.0f * s;
+#pragma unroll
+    for (int k = 1; k >= -1; k--) {
+      const float c = mid + (float)k * s;
+      p = plane_t(r.o[a], r.inv[a], c) >= from ? c : p;
+    }
+    p = (p - first) * s > 0.0f ? p : first;
+    w.cell[a] = (int32_t)p - r.pos[a];
+  }
+}
+
+// What the lane of a part walks of a ray that walk_dense() takes: its start in
+// w and the t it ends at in tmax; false when that is nothing.
+// The stretch may be empty or run backwards: the origin of a shadow ray is a
+// hit point, which rounding can leave beyond the very side of the grid that
+// the ray leaves by (t_out < 0), the more the farther the eye.  walk() then
+// reads the start cell and ends, and so does the first lane; a part's `from`
+// would lie past t_out, and its start cell past the grid.
+__device__ __forceinline__ bool dense_part(const DevScene &s, const Ray &r, const DenseRay &e,
+                                           WalkState &w, float &tmax, uint32_t part) {
+  const float t_lim = tmax < e.t_out ? tmax : e.t_out;
+  const float step = (t_lim - w.t) * (1.0f / kDenseParts);
+  if (!(step > 0.0f)) return part == 0u;
+  const float from = w.t + step * (float)part;  // at most t_lim: 3/4 of the stretch, rounded
+  if (part + 1u < (uint32_t)kDenseParts) {
+    const float to = w.t + step * (float)(part + 1u);
+    tmax = to < tmax ? to : tmax;
+  }
+  if (part > 0u) dense_skip(r, w, from);
+  // only planes with a t below t_out were crossed, so the cell is in the grid;
+  // walk_dense() reads it without a test, so it is tested here
+  bool in = true;
+#pragma unroll
+  for (int a = 0; a < 3; a++) in = in && (uint32_t)w.cell[a] < (uint32_t)s.n;
+  return in;
+}
+
+// walk() by the four lanes of a pixel: true in those that hit.  A start cell
+// that is solid was the last cell of the part before, whose lane then has it.
+__device__ __forceinline__ bool walk_part(const DevScene &s, const Ray &r, WalkState &w, float tmax,
+                                          uint32_t part, uint16_t &material) {
+  if (!(w.t < tmax)) return false;
+  DenseRay e;
+  if (!e.setup(s, r)) {
+    StepCounts cnt;
+    return part == 0u && walk<1, false>(s, r, w, tmax, material, cnt);
+  }
+  return dense_part(s, r, e, w, tmax, part) && walk_dense<kDenseAhead>(s, r, e, w, tmax, material);
+}
+
 __device__ __forceinline__ void primary_ray(const DevCamera &c, int32_t px, int32_t py, float o[3],
                                             float d[3]) {
   float a = (float)px + 0.5f;

@@ -1,0 +1,86 @@
+"""Eyes so far off that rounding puts hit points, and with them the origins of
+shadow and occlusion rays, outside the scene, against the oracle.
+
+Dense: frames whose pixels are a few thousandths of a voxel and less, at the
+edge of a slab at either end of the grid, with the light toward that end, so
+that shadow rays start beyond the plane they leave by (counted on the CPU).
+The default launch, 8x8 tiles (four lanes a ray both) and 16x16 tiles.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+from mesoengine_amd import _lib as L
+from mesoengine_amd import runtime as R
+
+from test_gpu_variants import _check, _force, _fresh
+
+pytestmark = pytest.mark.gpu
+
+
+def _beyond(ocam, ref, n, light):
+    """Lit hits whose point lies outside the grid on a side that the light is toward."""
+    w = ocam.width
+    count = 0
+    for pix in np.flatnonzero(ref[1] < 6):
+        f = int(ref[1][pix])
+        axis = 2 - f // 2
+        sign = -1 if f & 1 else 1
+        if light[axis] * sign <= 0:
+            continue
+        o, d = O.primary_ray(ocam, int(pix % w), int(pix // w))
+        p = o + d * ref[2][pix]
+        i = int(ref[0][pix])
+        start = [i % n, i // n % n, i // n // n]
+        start[axis] += sign
+        if all(0 <= c < n for c in start):
+            count += any((p[a] < 0 and light[a] < 0) or (p[a] > n and light[a] > 0)
+                         for a in range(3))
+    return count
+
+
+def dense_edge(n, axis, up_axis, high, dist, rng):
+    """A slab up to the middle of `up_axis`, an eye and a light for its edge at the
+    low or high end of `axis`."""
+    sl = [slice(None)] * 3
+    sl[2 - up_axis] = slice(0, n // 2)
+    grid = np.zeros((n, n, n), np.uint8)  # (z, y, x)
+    grid[tuple(sl)] = 2
+    target, direction, light = [n * 0.43] * 3, [0.17] * 3, [0.11] * 3
+    target[axis], target[up_axis] = (n if high else 0.0), n // 2
+    direction[axis], direction[up_axis] = (-0.6 if high else 0.6), 0.7
+    light[axis], light[up_axis] = (0.6 if high else -0.6), 0.8
+    eye = [float(np.float32(t + dist * (c + 0.3 * (j - 0.5))))
+           for t, c, j in zip(target, direction, rng.random(3))]
+    up = [0.0, 0.0, 0.0]
+    up[3 - axis - up_axis] = 1.0
+    return grid, eye, target, up, light
+
+
+# a hit point lies beyond a side when its plane and the side's plane are crossed
+# at one t, where the axes' order enters the voxel first: axis after up_axis
+@pytest.mark.parametrize("dist", [3000.0, 60000.0])
+@pytest.mark.parametrize("high", [0, 1])
+@pytest.mark.parametrize("axis,up_axis", [(1, 0), (2, 0), (2, 1)])
+@pytest.mark.parametrize("n", [16, 63])
+def test_dense_shadow_rays_from_beyond_the_grid(ctx, tmp_path, n, axis, up_axis, high, dist):
+    rng = np.random.default_rng(7)
+    w, h, flags, beyond = 57, 41, L.RAY_SHADOW, 0
+    fov = float(np.degrees(300 * 2.0 ** -24 * h))  # some 300 roundings of the distance a pixel
+    tg = R.RayTargets(ctx, w, h)
+    for frame in range(8):
+        grid, eye, target, up, light = dense_edge(n, axis, up_axis, high, dist, rng)
+        view = (eye, target, up, fov, w, h)
+        ocam, sh = O.camera(*view), (light, 3, 4, 5.0)
+        ref = O.raymarch(O.dense_scene(grid.ravel()), ocam, flags, O.shading(*sh), threads=4)
+        beyond += _beyond(ocam, ref, n, light)
+        sc = ctx.scene_dense(grid)
+        for shape in [None, (0, 16, 16, 0), (2, 8, 8, 0)]:
+            if shape:
+                _force(ctx, tmp_path, L.SCENE_DENSE_U8, n, w, h, flags, shape)
+            _fresh(tg)
+            R.raymarch(ctx, sc, R.camera(*view), flags, R.shading(*sh), tg)
+            ctx.sync()
+            _check(ctx, tg, ref, "n=%d axis %d %s" % (n, axis, shape), count=False)
+        sc.destroy()
+    assert beyond > 0
