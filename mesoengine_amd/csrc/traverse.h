@@ -529,15 +529,19 @@ __device__ __forceinline__ bool walk_bricks(const DevScene &s, const Ray &r, Wal
   const int32_t n = s.n;
   const uint32_t n128 = (uint32_t)(n + 127) >> 7, n32 = (uint32_t)(n + 31) >> 5;
   int32_t um[3], beyond[3];
-  float t_lim = tmax;
+  float o[3], t_lim = tmax;
 #pragma unroll
   for (int a = 0; a < 3; a++) {
     um[a] = r.up[a] ? -1 : 0;
     asm("" : "+v"(um[a]));  // a value, not a select again at each use
-    // an axis the ray does not move along: a plane above every origin
+    // An axis the ray does not move along: a plane 2^20 above the cell, and the
+    // origin at most 2^19, so that its t is +inf.  (A hit point of an eye that
+    // is 2^44 voxels away may lie farther off; cells are clamped to the scene,
+    // 8192 at most, so the step sees no difference.)
     beyond[a] = r.step[a] > 0 ? 1 : (r.step[a] < 0 ? 0 : 1 << 20);
+    o[a] = r.step[a] == 0 && r.o[a] > 524288.0f ? 524288.0f : r.o[a];
     const float far = r.step[a] > 0 ? s.fhi[a] : s.flo[a];
-    const float t = plane_t(r.o[a], r.inv[a], r.step[a] == 0 ? __builtin_inff() : far);
+    const float t = plane_t(o[a], r.inv[a], r.step[a] == 0 ? __builtin_inff() : far);
     t_lim = fminf(t_lim, t);
   }
   int32_t cx = w.cell[0], cy = w.cell[1], cz = w.cell[2];
@@ -592,12 +596,12 @@ __device__ __forceinline__ bool walk_bricks(const DevScene &s, const Ray &r, Wal
     const int32_t b0 = (um[0] & span) | (cx & ~span), b1 = (um[1] & span) | (cy & ~span),
                   b2 = (um[2] & span) | (cz & ~span);
     const int32_t p0 = b0 + beyond[0], p1 = b1 + beyond[1], p2 = b2 + beyond[2];
-    const float t0 = plane_t(r.o[0], r.inv[0], (float)p0), t1 = plane_t(r.o[1], r.inv[1], (float)p1),
-                t2 = plane_t(r.o[2], r.inv[2], (float)p2);
+    const float t0 = plane_t(o[0], r.inv[0], (float)p0), t1 = plane_t(o[1], r.inv[1], (float)p1),
+                t2 = plane_t(o[2], r.inv[2], (float)p2);
     const bool a0 = (t0 <= t1) & (t0 <= t2), a1 = !a0 & (t1 <= t2), a2 = !a0 & !a1;  // argmin3
     const float t = a0 ? t0 : (a1 ? t1 : t2);
     const float d0 = r.d[0] * t, d1 = r.d[1] * t, d2 = r.d[2] * t;
-    const float q0 = r.o[0] + d0, q1 = r.o[1] + d1, q2 = r.o[2] + d2;
+    const float q0 = o[0] + d0, q1 = o[1] + d1, q2 = o[2] + d2;
     const int32_t h0 = b0 > n - 1 ? n - 1 : b0, h1 = b1 > n - 1 ? n - 1 : b1,
                   h2 = b2 > n - 1 ? n - 1 : b2;
     const int32_t c0 = med3_i32(floor_i32(q0), cx, h0), c1 = med3_i32(floor_i32(q1), cy, h1),

@@ -84,3 +84,43 @@ def test_dense_shadow_rays_from_beyond_the_grid(ctx, tmp_path, n, axis, up_axis,
             _check(ctx, tg, ref, "n=%d axis %d %s" % (n, axis, shape), count=False)
         sc.destroy()
     assert beyond > 0
+
+
+# An eye 2^46 voxels away and more: the few directions that hit the scene put
+# the hit point millions of voxels off, also along an axis that the light has no
+# part in, on which shadow rays then do not move (counted on the CPU).
+@pytest.mark.parametrize("kind", [L.SCENE_BRICKMAP_U16, L.SCENE_TWO_LEVEL_U16])
+def test_brick_shadow_rays_from_far_off_an_axis(ctx, kind):
+    n, w, h, flags = 128, 9, 8, L.RAY_SHADOW | L.RAY_AO
+    grid = np.zeros((n, n, n), np.uint16)
+    grid[np.random.default_rng(3).random((n, n, n)) < 0.2] = 3
+    bricks = O.brickmap_from_dense(grid)
+    if kind == L.SCENE_BRICKMAP_U16:
+        sc, osc = ctx.scene_brickmap(n, *bricks), O.brickmap_scene(n, *bricks)
+    else:
+        nodes = O.two_level_from_bricks(n, *bricks)
+        sc, osc = ctx.scene_two_level(n, *nodes), O.two_level_scene(n, *nodes)
+    tg = R.RayTargets(ctx, w, h, index_bytes=8)
+    far = 0
+    for e, seed in [(e, seed) for e in (46, 50, 52) for seed in range(30)]:
+        d = np.random.default_rng(seed).normal(size=3)
+        eye = [float(np.float32(c * 2.0 ** e)) for c in d / np.linalg.norm(d)]
+        view = (eye, (n / 2.0,) * 3, (0.1, 1.0, 0.2), 1e-6, w, h)
+        ocam = O.camera(*view)
+        for light in [(0.0, 1.0, 0.0), (1.0, 0.0, 0.0), (0.0, 0.0, -1.0), (0.0, -1.0, 0.0)]:
+            ref = O.raymarch(osc, ocam, flags, O.shading(light, 1, 4, 5.0))
+            hits = np.flatnonzero(ref[1] < 6)
+            if not len(hits):
+                break
+            for pix in hits:
+                o, dd = O.primary_ray(ocam, int(pix % w), int(pix // w))
+                p = o + dd * ref[2][pix]
+                axis, sign = 2 - ref[1][pix] // 2, -1 if ref[1][pix] & 1 else 1
+                far += light[axis] * sign > 0 and any(light[a] == 0 and p[a] > 2 ** 20 + n
+                                                      for a in range(3))
+            _fresh(tg)
+            R.raymarch(ctx, sc, R.camera(*view), flags, R.shading(light, 1, 4, 5.0), tg)
+            ctx.sync()
+            _check(ctx, tg, ref, "2^%d seed %d light %s" % (e, seed, light), count=False)
+    sc.destroy()
+    assert far > 0

@@ -69,3 +69,8 @@ def _run(walks, *args):
 @pytest.mark.parametrize("seed", [1, 2])
 def test_parts_of_dense_rays(walks, seed):
     _run(walks, "dense", seed, 1_500_000)
+
+
+@pytest.mark.parametrize("seed", [1, 2])
+def test_secondary_rays_of_brick_scenes(walks, seed):
+    _run(walks, "bricks", seed, 3_000_000)
