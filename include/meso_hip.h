@@ -528,6 +528,11 @@ typedef struct meso_raster_stats {
 meso_status meso_raster_create(meso_context *ctx, int32_t max_width, int32_t max_height,
                                meso_raster **out);
 meso_status meso_raster_destroy(meso_raster *raster);
+/* Lowers what the lists hold: quads (records) and pixel tests (windows of 256).
+ * The default, and the most, is what meso_raster_create allocates.  Quads that
+ * find no room are tested where they are found, with the same result, so the
+ * limits change times only; tests use it to reach that path with few quads. */
+meso_status meso_raster_set_list_limits(meso_raster *raster, uint32_t records, uint32_t windows);
 /* One frame of the pool's resident quads; runs on `stream` without a host
  * wait.  Calls on one raster object must be ordered. */
 meso_status meso_raster_pool(meso_raster *raster, meso_chunk_pool *pool, const meso_camera *cam,

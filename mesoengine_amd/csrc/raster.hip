@@ -30,18 +30,17 @@
 // one FP32 operation at a time, as in the oracle, and uses the raymarcher's
 // primary ray and its plane distance (p - o) * (1 / d), so t equals the DDA's
 // entry t bit for bit when both find the same face.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 
+#include "raster_lists.h"
 #include "traverse.h"
 
 namespace meso {
 
 constexpr uint32_t kPoolNoSlot = 0xFFFFFFFFu;
 constexpr int kSmall = 64;           // counted apart in the stats
-constexpr uint32_t kWindow = 256u;   // pixel tests per window
-constexpr uint32_t kMaxWindows = 1u << 23;
-constexpr uint32_t kMaxRecords = 1u << 22;
 constexpr uint32_t kMaxItems = 1u << 22;
 
 __device__ __forceinline__ void chunk_origin(uint32_t chunk, uint32_t nc, int32_t o[3]) {
@@ -281,9 +280,9 @@ struct RasterScratch {
   // lowest [0] at which something did not fit; of the frame: [2] small | large
   // << 32 quads, [3] records | overflowed quads << 32
   unsigned long long *counters;
+  ListLimits limits;
 };
 enum : int { kRasterTests = 0, kRasterItems = 1, kRasterDrawn = 2, kRasterRecords = 3, kRasterFull = 4, kRasterCounters = 5 };
-constexpr uint64_t kTestsMask = (1ull << 40) - 1ull, kMaxTests = (uint64_t)kMaxWindows * kWindow;
 
 // Farthest t (as float bits; ~0 where a pixel has no hit yet) of the blocks of
 // 8, 32 and 128 pixels.
@@ -453,12 +452,13 @@ __device__ __forceinline__ QuadGeom unpack_geom(uint32_t b0, uint32_t b1) {
 // a workgroup adds once per kCollect quads or more (an add per wave and 64
 // quads took 0.79 ms for the far shell of 16,384 cave chunks, this 0.15 ms).
 constexpr uint32_t kQuadThreads = 512u, kCollect = 512u;
+static_assert(2u * kCollect <= kMaxLot, "a lot");
 struct Collected {
   uint32_t id[2 * kCollect], xy[2 * kCollect], rw[2 * kCollect], area[2 * kCollect];
   uint2 geom[2 * kCollect];
   uint64_t wave_sum[kQuadThreads / 64];
-  uint32_t wave_n[kQuadThreads / 64];
   uint32_t n;
+  bool full;  // a lot did not fit: the workgroup tests the rest of its quads itself
   unsigned long long at;
 };
 
@@ -485,16 +485,13 @@ __device__ __forceinline__ void flush_quads(Collected &C, const DevCamera &cam,
     all += C.wave_sum[w];
   }
   if (t == 0) {
-    // an outsized lot is not added: the counts of all workgroups in flight
-    // stay inside their fields (1024 workgroups * 2^28 tests, 2^10 records)
-    C.at = all > kMaxTests / 8u
-               ? ~0ull
-               : atomicAdd(&s.counters[kRasterTests], all | ((unsigned long long)n << 40));
+    const uint64_t add = lot_word(s.limits, n, all, C.full);
+    C.at = add ? atomicAdd(&s.counters[kRasterTests], (unsigned long long)add) : ~0ull;
   }
   __syncthreads();
   const unsigned long long at = C.at;
   const uint64_t rec0 = at >> 40, test0 = at & kTestsMask;
-  if (rec0 + n <= kMaxRecords && test0 + all <= kMaxTests) {  // uniform
+  if (at != ~0ull && lot_fits(s.limits, at, n, all)) {  // uniform
     uint64_t start = test0 + before;
 #pragma unroll
     for (uint32_t j = 0; j < 2u; j++) {
@@ -520,17 +517,22 @@ __device__ __forceinline__ void flush_quads(Collected &C, const DevCamera &cam,
     }
     if (t == 0) n_records += n;
   } else {
-    // no room: the workgroup tests its quads' pixels here.  Everything added
-    // after the first that did not fit does not fit either (both counts only
-    // grow), so raster_pixels_kernel stops there.
-    if (t == 0 && at != ~0ull) atomicMin(&s.counters[kRasterFull], at);
+    // no room: the workgroup tests its quads' pixels here, a wave per quad, or
+    // all of it where they are large.  raster_pixels_kernel stops at the first
+    // lot that did not fit.
+    if (t == 0 && at != ~0ull) {
+      atomicMin(&s.counters[kRasterFull], at);
+      C.full = true;
+    }
     if (t == 0) n_over += n;
     const uint64_t npx = (uint64_t)cam.width * (uint32_t)cam.height;
     const float eye[3] = {cam.eye[0], cam.eye[1], cam.eye[2]};
-    for (uint32_t q = 0; q < n; q++) {
+    const bool wide = all > (uint64_t)n * kQuadThreads;
+    const uint32_t q_step = wide ? 1u : kQuadThreads / 64u, p_step = wide ? kQuadThreads : 64u;
+    for (uint32_t q = wide ? 0u : wave; q < n; q += q_step) {
       const QuadGeom g = unpack_geom(C.geom[q].x, C.geom[q].y);
       const uint32_t xy = C.xy[q], w = C.rw[q], a = C.area[q];
-      for (uint32_t p = t; p < a; p += kQuadThreads)
+      for (uint32_t p = wide ? t : lane; p < a; p += p_step)
         test_pixel(g, eye, (uint64_t)((xy >> 14) + p / w) * (uint32_t)cam.width + (xy & 0x3FFFu) + p % w,
                    npx, C.id[q], s);
     }
@@ -554,7 +556,10 @@ __global__ void __launch_bounds__(kQuadThreads, 5) raster_quads_kernel(
   const uint32_t n_items = (uint32_t)s.counters[kRasterItems];
   const float eye[3] = {cam.eye[0], cam.eye[1], cam.eye[2]};
   uint32_t n_small = 0, n_large = 0, n_records = 0, n_over = 0;
-  if (threadIdx.x == 0) C.n = 0u;
+  if (threadIdx.x == 0) {
+    C.n = 0u;
+    C.full = false;
+  }
   __syncthreads();
   // every wave of the workgroup makes the same trips
   for (uint32_t it0 = blockIdx.x * kWaves; it0 < n_items; it0 += gridDim.x * kWaves) {
@@ -830,6 +835,7 @@ meso_status meso_raster_create(meso_context *ctx, int32_t max_width, int32_t max
   r->ctx = ctx;
   r->max_width = max_width;
   r->max_height = max_height;
+  r->s.limits = ListLimits{kMaxRecords, kMaxTests};
   const uint64_t npx = (uint64_t)max_width * (uint64_t)max_height;
   const DepthLevels d = depth_levels(nullptr, max_width, max_height);
   const uint64_t depth = (uint64_t)d.at128 + (uint64_t)d.w128 * ((uint32_t)(max_height + 127) / 128u);
@@ -846,6 +852,13 @@ meso_status meso_raster_create(meso_context *ctx, int32_t max_width, int32_t max
     return fail(MESO_ERR_OUT_OF_MEMORY, "raster: cannot allocate its scratch");
   }
   *out = r;
+  return MESO_OK;
+}
+
+meso_status meso_raster_set_list_limits(meso_raster *r, uint32_t records, uint32_t windows) {
+  MESO_CHECK(r, MESO_ERR_ARGUMENT_OUT_OF_RANGE, "NULL argument");
+  r->s.limits = ListLimits{std::min(records, kMaxRecords),
+                           (uint64_t)std::min(windows, kMaxWindows) * kWindow};
   return MESO_OK;
 }
 
@@ -920,7 +933,7 @@ meso_status meso_raster_pool(meso_raster *r, meso_chunk_pool *pool, const meso_c
                        v, pv.slot_chunk, pv.slot_count, cap, per, (uint32_t)pv.nc, batch,
                        bound[k] * bound[k], bound[k + 1] * bound[k + 1], k > 0, depth, r->s);
     MESO_HIP(hipGetLastError());
-    hipLaunchKernelGGL(raster_quads_kernel, dim3(waves / 8u), dim3(kQuadThreads), 0, s, dc, v, pv.slot_chunk,
+    hipLaunchKernelGGL(raster_quads_kernel, dim3(std::min(waves / 8u, kMaxLotGroups)), dim3(kQuadThreads), 0, s, dc, v, pv.slot_chunk,
                        pv.slot_count, pv.quads, per, (uint32_t)pv.nc, batch, k > 0, depth, r->s);
     MESO_HIP(hipGetLastError());
     hipLaunchKernelGGL(raster_pixels_kernel, dim3(2u * waves), dim3(64), 0, s, dc, r->s);
