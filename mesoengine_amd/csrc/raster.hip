@@ -320,11 +320,15 @@ __device__ __forceinline__ bool hidden(const DepthLevels &d, const int32_t r[4],
   return __float_as_uint(near) > m;
 }
 
+// The squared distance, finite: an eye 2^64 voxels away, whose distance is a
+// float but its square is not, counts as at the largest.
+__device__ __forceinline__ float square_dist(const float d[3]) {
+  return fminf(d[0] * d[0] + d[1] * d[1] + d[2] * d[2], 3.402823466e38f);
+}
 // A bound below the t of every hit on the box [lo, lo + size] from the eye:
 // its distance, less what the hit's rounding and the unit ray's can take off.
 __device__ __forceinline__ float near_bound(const float d[3]) {
-  const float q = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-  return __builtin_sqrtf(q) * 0.9999f - 0.01f;
+  return __builtin_sqrtf(square_dist(d)) * 0.9999f - 0.01f;
 }
 __device__ __forceinline__ float interval_gap(float e, float lo, float hi) {
   return fmaxf(fmaxf(lo - e, e - hi), 0.0f);
@@ -375,7 +379,7 @@ __global__ void __launch_bounds__(1024) raster_list_kernel(
 #pragma unroll
       for (int a = 0; a < 3; a++)
         d[a] = interval_gap(cam.eye[a], (float)o[a], (float)(o[a] + 32));
-      const float q = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+      const float q = square_dist(d);
       if (q >= near2 && q < far2) {
         int32_t r[4];
         const int in = chunk_view(cam, view, o, r);

@@ -124,3 +124,29 @@ def test_brick_shadow_rays_from_far_off_an_axis(ctx, kind):
             _check(ctx, tg, ref, "2^%d seed %d light %s" % (e, seed, light), count=False)
     sc.destroy()
     assert far > 0
+
+
+# An eye whose squared distance is above the largest float, looking along x: one
+# ray hits a slab's side all the same.  And one just below it.
+@pytest.mark.parametrize("dist", [1e18, 1.8e19, 1e20, 3e38])
+def test_quads_seen_from_beyond_the_squares(ctx, dist):
+    g = np.zeros((64, 64, 64), np.uint16)  # (z, y, x)
+    g[:, :8, :] = 1
+    sc = ctx.scene_brickmap(64, *O.brickmap_from_dense(g))
+    pool = R.ChunkPool(ctx, sc, capacity=8, quads_per_slot=1024, forward_radius=4,
+                       backward_radius=4, view_angle=120.0, max_loads=8)
+    pool.update((1, 1, 1), (1.0, 0.0, 0.0))
+    st = pool.state()
+    rast, tg = R.Raster(ctx, 3, 3), R.RayTargets(ctx, 1, 1)
+    eye = (float(np.float32(dist)), 4.5, 20.5)
+    view = (eye, (eye[0] * 0.999, 4.5, 20.5), (0.0, 1.0, 0.0), 40.0, 1, 1)
+    ref = O.raster_pool(O.camera(*view), 64, 2, st["slot_chunk"], st["slot_count"], st["quads"], 1024,
+                        O.shading((0.5, 1.0, 0.3)).light)
+    assert (ref[1][0] == 4) == (dist < 1e38)  # (at 3e38 the camera has no direction)
+    rast.draw(pool, R.camera(*view), R.shading((0.5, 1.0, 0.3)), tg)
+    ctx.sync()
+    for got, want in zip(tg.results(), ref[:4]):
+        assert np.array_equal(got.view(np.uint8), want.view(np.uint8))
+    rast.destroy()
+    pool.destroy()
+    sc.destroy()
