@@ -216,7 +216,7 @@ void free_scene_arrays(meso_scene *sc);
 meso_status launch_raymarch(meso_context *ctx, const meso_scene *scene, const DevCamera &cam,
                             uint32_t flags, const DevShading &sh, const RayOut &out,
                             hipStream_t stream, const RayLaunch *shape);
-RayLaunch default_ray_launch(const meso_scene *scene);
+RayLaunch default_ray_launch(bool count);
 meso_status launch_mesh_batched(meso_context *ctx, const meso_chunk_source *src, uint32_t mode,
                                 uint32_t *d_counts, uint32_t *d_prefix, uint32_t *d_quads,
                                 uint64_t capacity, uint64_t *d_total, void *d_work,

@@ -461,15 +461,19 @@ static meso_status launch_kind(meso_context *ctx, const meso_scene *scene, const
 // soon as its own 8x8 pixels are done, not the slowest of four packets.
 // 1920x1080 hills 170 us against 179 with 16x16 tiles, 3840x2160 caves 1936
 // against 1950; persistent waves 2036 there, and some 200 us more on the
-// smallest frames.
-RayLaunch default_ray_launch(const meso_scene *) { return RayLaunch{2, 64, 8, 8, 0}; }
+// smallest frames.  A launch that counts steps adds eleven counters to memory
+// per workgroup, on words that all of them share, and keeps the four packets
+// (1280x720 over 128^3 hills 228 us with 8x8 tiles, 119 with 16x16).
+RayLaunch default_ray_launch(bool count) {
+  return count ? RayLaunch{0, 256, 16, 16, 0} : RayLaunch{2, 64, 8, 8, 0};
+}
 
 meso_status launch_raymarch(meso_context *ctx, const meso_scene *scene, const DevCamera &cam,
                             uint32_t flags, const DevShading &sh, const RayOut &out,
                             hipStream_t stream, const RayLaunch *shape) {
-  const int variant = shape ? shape->variant : default_ray_launch(scene).variant;
-  const int grid = shape ? shape->grid : 0;
   const bool count = (flags & MESO_RAY_COUNT) != 0;
+  const int variant = shape ? shape->variant : default_ray_launch(count).variant;
+  const int grid = shape ? shape->grid : 0;
   switch (scene->kind) {
     case MESO_SCENE_DENSE_U8:
       return count ? launch_kind<1, true>(ctx, scene, cam, flags, sh, out, stream, variant, grid)

@@ -214,7 +214,7 @@ meso_status meso_autotune_raymarch(meso_context *ctx, meso_scene *scene, const m
         &st);
     if (st != MESO_OK) return st;
     tried++;
-    if (sp.v == default_ray_launch(scene).variant) best.default_ms = ms;
+    if (sp.v == default_ray_launch(false).variant) best.default_ms = ms;
     if (ms < best.best_ms) {
       best.best_ms = ms;
       best.variant = sp.v;
