@@ -533,6 +533,10 @@ meso_status meso_raster_destroy(meso_raster *raster);
  * find no room are tested where they are found, with the same result, so the
  * limits change times only; tests use it to reach that path with few quads. */
 meso_status meso_raster_set_list_limits(meso_raster *raster, uint32_t records, uint32_t windows);
+/* Resident chunks times pixels above which a frame is drawn in shells of chunks,
+ * the farther ones tested against what the nearer ones drew (default 2^32).
+ * The result is the same either way. */
+meso_status meso_raster_set_shell_line(meso_raster *raster, uint64_t chunk_pixels);
 /* One frame of the pool's resident quads; runs on `stream` without a host
  * wait.  Calls on one raster object must be ordered. */
 meso_status meso_raster_pool(meso_raster *raster, meso_chunk_pool *pool, const meso_camera *cam,

@@ -197,6 +197,7 @@ _SIGS = {
     "meso_chunk_pool_arrays": (C.c_int32, [P, P]),
     "meso_raster_create": (C.c_int32, [P, C.c_int32, C.c_int32, PP]),
     "meso_raster_destroy": (C.c_int32, [P]),
+    "meso_raster_set_shell_line": (C.c_int32, [P, C.c_uint64]),
     "meso_raster_set_list_limits": (C.c_int32, [P, C.c_uint32, C.c_uint32]),
     "meso_raster_pool": (C.c_int32, [P, P, P, P, P, P]),
     "meso_raster_stats_get": (C.c_int32, [P, P, P]),

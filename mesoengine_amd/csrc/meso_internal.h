@@ -198,6 +198,7 @@ struct PoolView {
   const meso_scene *scene;
   const uint32_t *slot_chunk, *slot_count, *quads;
   int32_t capacity, per_slot, nc;
+  uint32_t resident;  // at most so many slots hold a chunk (see meso_chunk_pool)
 };
 PoolView pool_view(const meso_chunk_pool *pool);
 hipStream_t stream_of(meso_context *ctx, meso_stream s);

@@ -12,6 +12,7 @@
 //
 // Float expressions follow the same one-operation-at-a-time order as the
 // oracle (-ffp-contract=off), so the ranking is bit-identical to it.
+#include <atomic>
 #include <cmath>
 #include <cstring>  // before rocprim, whose texture iterator calls memset
 #include <vector>
@@ -707,6 +708,9 @@ struct meso_chunk_pool {
   PoolGeom geom{};
   uint64_t cube = 0;
   uint32_t limit = 0;  // pairs considered per update: min(max_loads, capacity, cube)
+  // What the updates called so far can have loaded.  (Updates that a graph
+  // replays are not counted: a guide for how work is split, no more.)
+  std::atomic<uint32_t> resident{0};
   uint32_t *lookup = nullptr, *slot_chunk = nullptr, *slot_stamp = nullptr,
            *slot_count = nullptr, *quads = nullptr, *counters = nullptr;
   uint64_t *cand = nullptr, *cand_sorted = nullptr, *vict = nullptr, *vict_sorted = nullptr;
@@ -773,7 +777,8 @@ static meso_status pool_alloc(meso_chunk_pool *p, void **ptr, uint64_t bytes) {
 namespace meso {
 PoolView pool_view(const meso_chunk_pool *p) {
   return PoolView{p->scene, p->slot_chunk, p->slot_count, p->quads, p->geom.capacity,
-                  p->desc.quads_per_slot, p->geom.nc};
+                  p->desc.quads_per_slot, p->geom.nc,
+                  p->resident.load(std::memory_order_relaxed)};
 }
 }  // namespace meso
 
@@ -972,6 +977,9 @@ meso_status meso_chunk_pool_update(meso_chunk_pool *pool, const int32_t camera_c
                        pool->vict_sorted, pool->limit, tab, pool->counters);
     MESO_HIP(hipGetLastError());
   }
+  const uint32_t held = pool->resident.load(std::memory_order_relaxed);
+  pool->resident.store(cap - held > pool->limit ? held + pool->limit : cap,
+                       std::memory_order_relaxed);
   return launch_mesh_slotted(pool->ctx, pool->scene, pool->load_xyz, pool->load_slot,
                              pool->counters + kCntLoads, (int32_t)pool->limit,
                              pool->desc.mesh_mode, pool->slot_count, pool->quads,

@@ -10,7 +10,8 @@
 // waiting for the one with the largest quad, and the pixels of loose
 // rectangles.  So, on the device and without a host round trip:
 //   raster_begin_kernel: clears the keys and writes every pixel's ray.
-//   For each shell of chunks around the eye, nearest first:
+//   For each shell of chunks around the eye, nearest first (one shell for few
+//   chunks or pixels):
 //     raster_list_kernel: a lane per slot; slots of this shell whose box
 //       projects into the frame and is not hidden by what the nearer shells
 //       drew are listed, in items of a few dozen quads.
@@ -815,6 +816,7 @@ using namespace meso;
 
 struct meso_raster {
   meso_context *ctx = nullptr;
+  uint64_t shell_line = 1ull << 32;  // chunks * pixels above which there are shells
   int32_t max_width = 0, max_height = 0;
   RasterScratch s{};
 };
@@ -863,6 +865,12 @@ meso_status meso_raster_set_list_limits(meso_raster *r, uint32_t records, uint32
   MESO_CHECK(r, MESO_ERR_ARGUMENT_OUT_OF_RANGE, "NULL argument");
   r->s.limits = ListLimits{std::min(records, kMaxRecords),
                            (uint64_t)std::min(windows, kMaxWindows) * kWindow};
+  return MESO_OK;
+}
+
+meso_status meso_raster_set_shell_line(meso_raster *r, uint64_t chunk_pixels) {
+  MESO_CHECK(r, MESO_ERR_ARGUMENT_OUT_OF_RANGE, "NULL argument");
+  r->shell_line = chunk_pixels;
   return MESO_OK;
 }
 
@@ -926,13 +934,23 @@ meso_status meso_raster_pool(meso_raster *r, meso_chunk_pool *pool, const meso_c
   hipLaunchKernelGGL(raster_begin_kernel, grid_1d((npx + 255) / 256), dim3(256), 0, s, dc, r->s, npx);
   MESO_HIP(hipGetLastError());
   const uint32_t waves = (uint32_t)r->ctx->props.multiProcessorCount * 16u;
-  // Shell bounds in voxels (3 and 8 chunks).  A shell costs about 40 us of
-  // launches and small kernels and saves the quads hidden by the nearer ones:
-  // two shells (at 112) took 355 us where three (64, 160) took 318, (64, 160,
-  // 320) 262, and these 254 (16,384 cave chunks at 1920x1080).
+  // Shell bounds in voxels (3 and 8 chunks).  A shell costs 17 us of launches
+  // and small kernels, 25 in frames of 3840x2160, and saves the quads hidden by
+  // the nearer ones: two shells (at 112) took 355 us where three (64, 160) took
+  // 318, (64, 160, 320) 262, and these 254 (16,384 cave chunks at 1920x1080).
+  // What is saved grows with the chunks and with the pixels that a hidden quad
+  // covers, so few chunks or small frames have one shell for all.  Cave chunks
+  // with one shell and with three: 512 at 1920x1080 146 us and 183, at 3840x2160
+  // 374 and 383; 2,048 at 640x360 96 and 146, at 1920x1080 247 and 233, at
+  // 3840x2160 648 and 485; 16,384 at 320x180 134 and 167, at 640x360 186 and
+  // 179, at 1920x1080 579 and 291.  The line lies where the two meet.
   constexpr int kShells = 3;
-  const float bound[kShells + 1] = {0.0f, 96.0f, 256.0f, INFINITY};
-  for (int k = 0; k < kShells; k++) {
+  constexpr float kBound[kShells + 1] = {0.0f, 96.0f, 256.0f, INFINITY};
+  constexpr float kAll[2] = {0.0f, INFINITY};
+  const bool many = pv.resident * npx > r->shell_line;
+  const int shells = many ? kShells : 1;
+  const float *bound = many ? kBound : kAll;
+  for (int k = 0; k < shells; k++) {
     hipLaunchKernelGGL(raster_list_kernel, dim3((cap + 1023u) / 1024u), dim3(1024), 0, s, dc,
                        v, pv.slot_chunk, pv.slot_count, cap, per, (uint32_t)pv.nc, batch,
                        bound[k] * bound[k], bound[k + 1] * bound[k + 1], k > 0, depth, r->s);
@@ -942,7 +960,7 @@ meso_status meso_raster_pool(meso_raster *r, meso_chunk_pool *pool, const meso_c
     MESO_HIP(hipGetLastError());
     hipLaunchKernelGGL(raster_pixels_kernel, dim3(2u * waves), dim3(64), 0, s, dc, r->s);
     MESO_HIP(hipGetLastError());
-    if (k + 1 < kShells) {
+    if (k + 1 < shells) {
       hipLaunchKernelGGL(raster_depth_kernel,
                          dim3(depth.w128, (uint32_t)(cam->height + 127) / 128u), dim3(1024), 0, s,
                          r->s.keys, cam->width, cam->height, depth, r->s.far_t);
