@@ -75,12 +75,13 @@ __global__ void __launch_bounds__(TW *TH) raymarch_kernel(DevScene s, DevCamera 
 // itself.  Here a ray's stretch of t is cut into four, and each lane walks one
 // of them; the first lane of the four that hits has the hit.  AO rays, which are
 // short, are dealt out instead, one sample in four to a lane.  The rays' set-up
-// is done four times.  256x256 pixels over 256^3 voxels with shadows, a long
-// view, 120 us, now 60; 318x318 over 77^3 with shadows and two AO rays 42 and 22.
+// is done four times.  256^3 voxels of spheres with shadows, a long view, a lane
+// a ray and four: 200x200 119 and 52 us, 256x256 122 and 95, 400x225 121 and 51.
 //
-// The most 8x8 waves per SIMD of a frame that goes this way: 640x360, 3.5 a
-// SIMD, takes 75 us instead of 119, but 800x600, 7.3 a SIMD, 112 instead of 103.
-constexpr uint32_t kSmallWaves = 4;
+// The most 8x8 waves per SIMD of a frame that goes this way.  400x225, 1.4 a
+// SIMD, gains as above and takes 5.8 us instead of 3.9 where all is solid; 512x512,
+// 4 a SIMD, takes 124 instead of 119, and 11 instead of 4.8 where all is solid.
+constexpr uint32_t kSmallWaves = 2;
 
 __global__ void __launch_bounds__(64) raymarch_dense_small_kernel(DevScene s, DevCamera cam,
                                                                   uint32_t flags, DevShading sh,
@@ -96,8 +97,10 @@ __global__ void __launch_bounds__(64) raymarch_dense_small_kernel(DevScene s, De
   WalkState w = {{0, 0, 0}, 0.0f, 0};
   uint16_t m = 0;
   bool hit = false;
-  if (valid && trace_begin(s, o, d, r, w))
-    hit = walk_part(s, r, w, __builtin_inff(), part, m);
+  if (valid && trace_begin(s, o, d, r, w)) {
+    m = dense_start(s, w);
+    hit = m ? part == 0u : walk_part(s, r, w, __builtin_inff(), part, m);
+  }
   // the first of the pixel's lanes that hit, in every lane of the pixel
   const uint32_t hits = (uint32_t)(__ballot(hit) >> quad) & 15u;
   const int src = (int)(quad + (hits ? (uint32_t)__builtin_ctz(hits) : 0u));

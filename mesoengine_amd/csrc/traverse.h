@@ -370,10 +370,18 @@ __device__ __forceinline__ int walk_step(const DevScene &s, const Ray &r, WalkSt
 // made exact, was 5 times slower, lanes in blocks and lanes in steps running
 // both ways in every trip.)
 constexpr int kDenseAhead = 16;
-// where registers are short: the serving kernel's 131 with 16 left 3 waves a
-// SIMD, 103 leave 4 (200 queued requests, none of them dense: 12,050 Mrays/s
-// with 16, 13,370 with 4 workgroups a CU, 12,880 with the 5 that fit with no
-// cells ahead, which contend for the claims)
+// Rays that end within a few cells (solid scenes, eyes in them, occlusion rays of
+// rough ones) would pay for 16 all the same, so a walk first looks at some cells
+// one by one.  256^3 voxels at 1920x1080, primary rays, then with shadow and four
+// AO rays: solid from within 34 us with batches alone, now 18 (17 where a lane
+// steps through advance()); half of the voxels solid 38 and 183, now 28 and 152
+// (25 and 129); a tenth of them 61 and 329 now (80 and 363 there).  4 cells: 31
+// and 169 for the half, 62 and 314 for the tenth; a batch of 4 and then of 8
+// instead: 30 and 137, but 323 us where hills take 261, the code of two sizes of
+// batches taking registers.
+constexpr int kDenseSingle = 8;
+// where registers are short: the serving kernel has 131 with 16, which leaves 3
+// waves a SIMD, and 96 with 4
 constexpr int kDenseAheadShort = 4;
 constexpr int32_t kDenseIndexed = 1625;  // 1625^3 < 2^32: 32-bit voxel indices
 
@@ -425,33 +433,46 @@ __device__ __forceinline__ float dense_step(const Ray &r, float plane[3], int &a
   return t;
 }
 
-template <int AHEAD>
-__device__ __forceinline__ bool walk_dense(const DevScene &s, const Ray &r, const DenseRay &e,
-                                           WalkState &w, float tmax, uint16_t &material) {
-  const uint32_t n = (uint32_t)s.n;
-  const float t_lim = tmax < e.t_out ? tmax : e.t_out;
-  const uint32_t posmask = r.posmask;
-  auto face = [posmask](int ax) {  // entry_face
-    return 4 - 2 * ax + (int32_t)((posmask >> ax) & 1u);
-  };
-  float plane[3];
-  uint32_t stride[3];
+// A walk of a dense grid, a batch of cells at a time.
+struct DenseWalk {
+  const DevScene &s;
+  const Ray &r;
+  const DenseRay &e;
+  float tmax, t_lim;
+  float plane[3], from[3];  // exit planes of the next cell, and of the batch's first
+  uint32_t stride[3], idx, solid;
+  bool on;
+
+  __device__ __forceinline__ DenseWalk(const DevScene &s_, const Ray &r_, const DenseRay &e_,
+                                       const WalkState &w, float tmax_)
+      : s(s_), r(r_), e(e_), tmax(tmax_), solid(0), on(true) {
+    const uint32_t n = (uint32_t)s.n;
+    t_lim = tmax < e.t_out ? tmax : e.t_out;
 #pragma unroll
-  for (int a = 0; a < 3; a++) {
-    plane[a] = (float)(w.cell[a] + r.pos[a]);
-    const uint32_t d = a == 0 ? 1u : (a == 1 ? n : n * n);
-    stride[a] = r.step[a] < 0 ? 0u - d : d;
+    for (int a = 0; a < 3; a++) {
+      plane[a] = from[a] = (float)(w.cell[a] + r.pos[a]);
+      const uint32_t d = a == 0 ? 1u : (a == 1 ? n : n * n);
+      stride[a] = r.step[a] < 0 ? 0u - d : d;
+    }
+    idx = (uint32_t)w.cell[0] + n * ((uint32_t)w.cell[1] + n * (uint32_t)w.cell[2]);
   }
-  uint32_t idx = (uint32_t)w.cell[0] + n * ((uint32_t)w.cell[1] + n * (uint32_t)w.cell[2]);
-  for (;;) {
-    const float from[3] = {plane[0], plane[1], plane[2]};
+  __device__ __forceinline__ int32_t face(int ax) const {  // entry_face
+    return 4 - 2 * ax + (int32_t)((r.posmask >> ax) & 1u);
+  }
+  __device__ __forceinline__ int32_t cell(int a) const { return (int32_t)plane[a] - r.pos[a]; }
+
+  // The next CELLS cells (0: one that is empty, unread): true when none is solid and
+  // the walk goes on behind them (w.t and w.face then are the next cell's).
+  template <int CELLS>
+  __device__ __forceinline__ bool batch(WalkState &w) {
+    constexpr int N = CELLS ? CELLS : 1;
+    from[0] = plane[0], from[1] = plane[1], from[2] = plane[2];
     const uint32_t first = idx;
-    uint32_t at[AHEAD];
-    bool on = true;
+    uint32_t at[N];
     float t = 0.0f;
     int ax = 0;
 #pragma unroll
-    for (int i = 0; i < AHEAD; i++) {
+    for (int i = 0; i < N; i++) {
       // cells past the walk's end are read as the batch's first cell, which is
       // its first solid one or empty
       at[i] = on ? idx : first;
@@ -459,42 +480,60 @@ __device__ __forceinline__ bool walk_dense(const DevScene &s, const Ray &r, cons
       idx += ax == 0 ? stride[0] : (ax == 1 ? stride[1] : stride[2]);
       on = on && t < t_lim;
     }
-    uint32_t solid = 0;
-    uint8_t v[AHEAD];
+    uint8_t v[N];
 #pragma unroll
-    for (int i = 0; i < AHEAD; i++) v[i] = s.dense[at[i]];
+    for (int i = 0; i < N; i++) v[i] = CELLS ? s.dense[at[i]] : 0;
+    solid = 0;
 #pragma unroll
-    for (int i = 0; i < AHEAD; i++) solid |= (v[i] ? 1u : 0u) << i;
-    bool hit = solid != 0u;
-    if (hit || !on) {
-      // the batch's steps once more, to the first solid cell for its t, face
-      // and cell, or to the planes that have the t the ray leaves at
-      plane[0] = from[0], plane[1] = from[1], plane[2] = from[2];
-      if (hit) {
-        for (uint32_t k = (uint32_t)__builtin_ctz(solid); k; k--) {
-          w.t = dense_step(r, plane, ax);
-          w.face = face(ax);
-        }
-      } else {
-        if (!(e.t_out < tmax) || !e.ties(r)) return false;
-        while (!hit) {
-          const float t_now = dense_step(r, plane, ax);
-          if (t_now > e.t_out || (t_now == e.t_out && ax >= e.axis)) return false;
-          if (t_now < e.t_out) continue;
-          w.t = t_now;
-          w.face = face(ax);
-          hit = s.dense[lin3((int32_t)plane[0] - r.pos[0], (int32_t)plane[1] - r.pos[1],
-                             (int32_t)plane[2] - r.pos[2], s.n)] != 0;
-        }
-      }
-#pragma unroll
-      for (int a = 0; a < 3; a++) w.cell[a] = (int32_t)plane[a] - r.pos[a];
-      material = s.dense[lin3(w.cell[0], w.cell[1], w.cell[2], s.n)];
-      return true;
-    }
+    for (int i = 0; i < N; i++) solid |= (v[i] ? 1u : 0u) << i;
+    if (solid != 0u || !on) return false;
     w.t = t;
     w.face = face(ax);
+    return true;
   }
+
+  // After the batch that ended the walk, its steps once more, to the first solid
+  // cell for its t, face and cell, or to the planes that have the t the ray
+  // leaves at.
+  __device__ __forceinline__ bool finish(WalkState &w, uint16_t &material) {
+    plane[0] = from[0], plane[1] = from[1], plane[2] = from[2];
+    int ax = 0;
+    if (solid) {
+      for (uint32_t k = (uint32_t)__builtin_ctz(solid); k; k--) {
+        w.t = dense_step(r, plane, ax);
+        w.face = face(ax);
+      }
+    } else {
+      if (!(e.t_out < tmax) || !e.ties(r)) return false;
+      bool hit = false;
+      while (!hit) {
+        const float t_now = dense_step(r, plane, ax);
+        if (t_now > e.t_out || (t_now == e.t_out && ax >= e.axis)) return false;
+        if (t_now < e.t_out) continue;
+        w.t = t_now;
+        w.face = face(ax);
+        hit = s.dense[lin3(cell(0), cell(1), cell(2), s.n)] != 0;
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < 3; a++) w.cell[a] = cell(a);
+    material = s.dense[lin3(w.cell[0], w.cell[1], w.cell[2], s.n)];
+    return true;
+  }
+};
+
+// SINGLE: cells looked at one by one first (see kDenseSingle), AHEAD: cells of
+// a batch.  EMPTY: the start cell is known to be empty and not read again.
+template <int SINGLE, int AHEAD, bool EMPTY>
+__device__ __forceinline__ bool walk_dense(const DevScene &s, const Ray &r, const DenseRay &e,
+                                           WalkState &w, float tmax, uint16_t &material) {
+  DenseWalk d(s, r, e, w, tmax);
+  bool more = true;
+  if constexpr (EMPTY) more = d.batch<0>(w);
+#pragma unroll 1
+  for (int k = 0; k < SINGLE && more; k++) more = d.batch<1>(w);
+  while (more) more = d.batch<AHEAD>(w);
+  return d.finish(w, material);
 }
 
 // (a ^ -1) + b in one instruction
@@ -633,14 +672,15 @@ __device__ __forceinline__ bool walk_bricks(const DevScene &s, const Ray &r, Wal
 
 // Walk until a solid voxel is entered (true), the ray leaves the scene or the
 // entry t reaches tmax (false).
-template <int KIND, bool COUNT>
+// EMPTY: the start cell of a dense grid is known to be empty.
+template <int KIND, bool COUNT, bool EMPTY = false>
 __device__ __forceinline__ bool walk(const DevScene &s, const Ray &r, WalkState &w, float tmax,
                                      uint16_t &material, StepCounts &cnt) {
   if (!(w.t < tmax)) return false;
   if constexpr ((KIND == 1 || KIND == kDenseShort) && !COUNT) {
     constexpr int ahead = KIND == 1 ? kDenseAhead : kDenseAheadShort;
     DenseRay e;
-    if (e.setup(s, r)) return walk_dense<ahead>(s, r, e, w, tmax, material);
+    if (e.setup(s, r)) return walk_dense<kDenseSingle, ahead, EMPTY>(s, r, e, w, tmax, material);
   }
   if constexpr ((KIND == 2 || KIND == 3) && !COUNT) return walk_bricks<KIND>(s, r, w, tmax, material);
   WalkCache c;
@@ -702,8 +742,11 @@ __device__ __forceinline__ bool dense_part(const DevScene &s, const Ray &r, cons
   return in;
 }
 
-// walk() by the four lanes of a pixel: true in those that hit.  A start cell
+// walk() by the four lanes of a pixel: true in the first of those that hit and
+// perhaps in others.  The first kDenseTogether cells are looked at by all four,
+// and most rays of solid or rough scenes end there.  A start cell of a part
 // that is solid was the last cell of the part before, whose lane then has it.
+constexpr int kDenseTogether = 8;
 __device__ __forceinline__ bool walk_part(const DevScene &s, const Ray &r, WalkState &w, float tmax,
                                           uint32_t part, uint16_t &material) {
   if (!(w.t < tmax)) return false;
@@ -712,7 +755,11 @@ __device__ __forceinline__ bool walk_part(const DevScene &s, const Ray &r, WalkS
     StepCounts cnt;
     return part == 0u && walk<1, false>(s, r, w, tmax, material, cnt);
   }
-  return dense_part(s, r, e, w, tmax, part) && walk_dense<kDenseAhead>(s, r, e, w, tmax, material);
+  DenseWalk d(s, r, e, w, tmax);
+  if (!d.batch<kDenseTogether>(w)) return d.finish(w, material);
+#pragma unroll
+  for (int a = 0; a < 3; a++) w.cell[a] = d.cell(a);
+  return dense_part(s, r, e, w, tmax, part) && walk_dense<0, kDenseAhead, false>(s, r, e, w, tmax, material);
 }
 
 __device__ __forceinline__ void primary_ray(const DevCamera &c, int32_t px, int32_t py, float o[3],
@@ -796,6 +843,13 @@ __device__ __forceinline__ bool trace_begin(const DevScene &s, const float o[3],
   return true;
 }
 
+// The cell a primary ray of a dense grid enters first, looked at before the walk
+// is set up: all there is to do where the grid's sides are solid or the eye is
+// (see kDenseSingle).
+__device__ __forceinline__ uint16_t dense_start(const DevScene &s, const WalkState &w) {
+  return w.t < __builtin_inff() ? s.dense[lin3(w.cell[0], w.cell[1], w.cell[2], s.n)] : 0;
+}
+
 // Clip to [0,n]^3, find the entry cell and walk.
 template <int KIND, bool COUNT>
 __device__ __forceinline__ bool trace(const DevScene &s, const float o[3], const float d[3],
@@ -809,7 +863,9 @@ __device__ __forceinline__ bool trace(const DevScene &s, const float o[3], const
   if (!trace_begin(s, o, d, r, w)) return false;
   const int32_t n = s.n;
   uint16_t m = 0;
-  if (!walk<KIND, COUNT>(s, r, w, __builtin_inff(), m, cnt)) return false;
+  constexpr bool first = (KIND == 1 || KIND == kDenseShort) && !COUNT;
+  if constexpr (first) m = dense_start(s, w);
+  if (m == 0 && !walk<KIND, COUNT, first>(s, r, w, __builtin_inff(), m, cnt)) return false;
   hit.index = lin3(w.cell[0], w.cell[1], w.cell[2], n);
   hit.face = w.face;
   hit.t = w.t;

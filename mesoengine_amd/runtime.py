@@ -308,7 +308,7 @@ class Event:
 class Server:
     """The continuous-batching server: requests are admitted by the HBM
     budget into `max_inflight` ring entries that one persistent kernel of
-    `workgroups_per_cu` workgroups of 4 waves per CU (0: all that fit) draws
+    `workgroups_per_cu` workgroups of 4 waves per CU (0: what fits, up to 4) draws
     8x8-pixel packets from."""
 
     def __init__(self, ctx, budget_bytes, max_pending=256, max_inflight=64, workgroups_per_cu=0,
