@@ -207,10 +207,11 @@ meso_status launch_zero(void *ptr, uint64_t bytes, hipStream_t stream);
 meso_status init_mesh_scratch(meso_context *ctx);
 // the persistent raymarch's band counters for `stream` (1 KiB, zeroed once)
 meso_status band_queue(meso_context *ctx, hipStream_t stream, unsigned int **out);
-// builds the empty-space levels (occ32/occ128 or node groups) of a brick scene
-meso_status build_coarse(meso_scene *sc, hipStream_t stream);
-// sets masks_match of a scene whose bricks came from the caller
-meso_status check_masks(meso_scene *sc, hipStream_t stream);
+// builds the empty-space levels (occ32/occ128 or node groups) of a brick scene;
+// uploaded: its bricks came from the caller, so masks_match is found out too
+meso_status build_coarse(meso_scene *sc, hipStream_t stream, bool uploaded);
+// sets *bad (device, zero before) where a brick's mask is not that of its voxels
+meso_status launch_mask_check(const meso_scene *sc, uint32_t *bad, hipStream_t stream);
 void free_scene_arrays(meso_scene *sc);
 
 // kernels launched by other translation units

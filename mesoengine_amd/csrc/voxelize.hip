@@ -624,7 +624,7 @@ __global__ void __launch_bounds__(512) edit_chunks_kernel(DevScene s, int32_t ki
   }
 }
 
-// Counts the bricks whose mask is not that of their voxels: a wave per brick.
+// *bad: whether some brick's mask is not that of its voxels.  A wave per brick.
 __global__ void __launch_bounds__(256) mask_check_kernel(const uint64_t *masks,
                                                          const uint16_t *voxels, uint64_t n_bricks,
                                                          uint32_t *bad) {
@@ -640,23 +640,12 @@ __global__ void __launch_bounds__(256) mask_check_kernel(const uint64_t *masks,
   if (__ballot(differs) && lane == 0) atomicOr(bad, 1u);
 }
 
-meso_status check_masks(meso_scene *sc, hipStream_t stream) {
-  sc->masks_match = true;
+meso_status launch_mask_check(const meso_scene *sc, uint32_t *bad, hipStream_t stream) {
   if (sc->n_bricks == 0) return MESO_OK;
-  uint32_t *bad = nullptr, host = 0;
-  MESO_HIP(hipMallocAsync((void **)&bad, 16, stream));
-  meso_status st = launch_zero(bad, 16, stream);
-  if (st == MESO_OK) {
-    hipLaunchKernelGGL(mask_check_kernel, grid_1d(((uint64_t)sc->n_bricks + 3) / 4), dim3(256), 0,
-                       stream, sc->masks, sc->voxels, (uint64_t)sc->n_bricks, bad);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(&host, bad, 4, hipMemcpyDeviceToHost, stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(stream);
-    if (e != hipSuccess) st = fail(MESO_ERR_RUNTIME, "mask check: %s", hipGetErrorString(e));
-  }
-  (void)hipFreeAsync(bad, stream);
-  sc->masks_match = host == 0;
-  return st;
+  hipLaunchKernelGGL(mask_check_kernel, grid_1d(((uint64_t)sc->n_bricks + 3) / 4), dim3(256), 0,
+                     stream, sc->masks, sc->voxels, (uint64_t)sc->n_bricks, bad);
+  MESO_HIP(hipGetLastError());
+  return MESO_OK;
 }
 
 }  // namespace meso
@@ -867,7 +856,7 @@ meso_status meso_scene_generate(meso_context *ctx, const meso_generate_desc *d, 
   (void)hipFreeAsync(scratch, stream);
   if (st != MESO_OK) return gen_free(sc, st);
   sc->masks_match = true;  // brick_write_kernel makes both from the same words
-  GEN_TRY(build_coarse(sc, stream));
+  GEN_TRY(build_coarse(sc, stream, false));
   *out = sc;
   return MESO_OK;
 }
