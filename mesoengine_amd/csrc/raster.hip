@@ -34,6 +34,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 #include "raster_lists.h"
 #include "traverse.h"
@@ -816,17 +817,11 @@ using namespace meso;
 
 struct meso_raster {
   meso_context *ctx = nullptr;
+  void *scratch = nullptr;  // holds the arrays of s
   uint64_t shell_line = 1ull << 32;  // chunks * pixels above which there are shells
   int32_t max_width = 0, max_height = 0;
   RasterScratch s{};
 };
-
-static void raster_free(meso_raster *r) {
-  for (void *p : {(void *)r->s.keys, (void *)r->s.rays, (void *)r->s.far_t, (void *)r->s.items,
-                  (void *)r->s.rec_a, (void *)r->s.rec_b, (void *)r->s.windows, (void *)r->s.counters})
-    if (p) (void)hipFree(p);
-  delete r;
-}
 
 extern "C" {
 
@@ -845,18 +840,32 @@ meso_status meso_raster_create(meso_context *ctx, int32_t max_width, int32_t max
   const uint64_t npx = (uint64_t)max_width * (uint64_t)max_height;
   const DepthLevels d = depth_levels(nullptr, max_width, max_height);
   const uint64_t depth = (uint64_t)d.at128 + (uint64_t)d.w128 * ((uint32_t)(max_height + 127) / 128u);
-  if (hipMalloc((void **)&r->s.keys, npx * 8) != hipSuccess ||
-      hipMalloc((void **)&r->s.rays, npx * 12) != hipSuccess ||
-      hipMalloc((void **)&r->s.far_t, depth * 4) != hipSuccess ||
-      hipMalloc((void **)&r->s.items, (uint64_t)kMaxItems * 4) != hipSuccess ||
-      hipMalloc((void **)&r->s.rec_a, (uint64_t)kMaxRecords * 16) != hipSuccess ||
-      hipMalloc((void **)&r->s.rec_b, (uint64_t)kMaxRecords * 8) != hipSuccess ||
-      hipMalloc((void **)&r->s.windows, (uint64_t)kMaxWindows * 4) != hipSuccess ||
-      hipMalloc((void **)&r->s.counters, kRasterCounters * 8) != hipSuccess) {
+  // one allocation, each array from a multiple of 256 bytes (one for each took
+  // 1.2 ms for frames of 1920x1080, this 0.29)
+  const uint64_t bytes[] = {npx * 8, npx * 12, depth * 4, (uint64_t)kMaxItems * 4,
+                            (uint64_t)kMaxRecords * 16, (uint64_t)kMaxRecords * 8,
+                            (uint64_t)kMaxWindows * 4, kRasterCounters * 8};
+  uint64_t total = 0;
+  for (uint64_t b : bytes) total += (b + 255u) & ~255ull;
+  if (hipMalloc(&r->scratch, total) != hipSuccess) {
     (void)hipGetLastError();
-    raster_free(r);
+    delete r;
     return fail(MESO_ERR_OUT_OF_MEMORY, "raster: cannot allocate its scratch");
   }
+  uint8_t *at = (uint8_t *)r->scratch;
+  int k = 0;
+  const auto take = [&](auto *&p) {
+    p = (std::remove_reference_t<decltype(p)>)at;
+    at += (bytes[k++] + 255u) & ~255ull;
+  };
+  take(r->s.keys);
+  take(r->s.rays);
+  take(r->s.far_t);
+  take(r->s.items);
+  take(r->s.rec_a);
+  take(r->s.rec_b);
+  take(r->s.windows);
+  take(r->s.counters);
   *out = r;
   return MESO_OK;
 }
@@ -877,7 +886,8 @@ meso_status meso_raster_set_shell_line(meso_raster *r, uint64_t chunk_pixels) {
 meso_status meso_raster_destroy(meso_raster *r) {
   if (!r) return MESO_OK;
   (void)hipDeviceSynchronize();
-  raster_free(r);
+  (void)hipFree(r->scratch);
+  delete r;
   return MESO_OK;
 }
 
