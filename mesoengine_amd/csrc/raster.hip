@@ -523,22 +523,21 @@ __device__ __forceinline__ void flush_quads(Collected &C, const DevCamera &cam,
     }
     if (t == 0) n_records += n;
   } else {
-    // no room: the workgroup tests its quads' pixels here, a wave per quad, or
-    // all of it where they are large.  raster_pixels_kernel stops at the first
-    // lot that did not fit.
-    if (t == 0 && at != ~0ull) {
-      atomicMin(&s.counters[kRasterFull], at);
-      C.full = true;
+    // no room: the workgroup tests its quads' pixels here, a wave per quad.
+    // raster_pixels_kernel stops at the first lot that did not fit.
+    if (t == 0) {
+      if (at != ~0ull) {
+        atomicMin(&s.counters[kRasterFull], at);
+        C.full = true;
+      }
+      n_over += n;
     }
-    if (t == 0) n_over += n;
     const uint64_t npx = (uint64_t)cam.width * (uint32_t)cam.height;
     const float eye[3] = {cam.eye[0], cam.eye[1], cam.eye[2]};
-    const bool wide = all > (uint64_t)n * kQuadThreads;
-    const uint32_t q_step = wide ? 1u : kQuadThreads / 64u, p_step = wide ? kQuadThreads : 64u;
-    for (uint32_t q = wide ? 0u : wave; q < n; q += q_step) {
+    for (uint32_t q = wave; q < n; q += kQuadThreads / 64u) {
       const QuadGeom g = unpack_geom(C.geom[q].x, C.geom[q].y);
       const uint32_t xy = C.xy[q], w = C.rw[q], a = C.area[q];
-      for (uint32_t p = wide ? t : lane; p < a; p += p_step)
+      for (uint32_t p = lane; p < a; p += 64u)
         test_pixel(g, eye, (uint64_t)((xy >> 14) + p / w) * (uint32_t)cam.width + (xy & 0x3FFFu) + p % w,
                    npx, C.id[q], s);
     }
