@@ -268,7 +268,8 @@ __device__ __forceinline__ int chunk_view(const DevCamera &c, const RasterView &
 }
 
 // One shell's pixel tests are numbered through: record i owns the tests from
-// its start to the next record's.  {start, quad id, x0 | y0 << 14, width} and
+// its start to the next record's.  {start, quad id, x0 | y0 << 14, width |
+// tests per row << 16} (tests_per_row) and
 // {U0 | V0 << 13 | face << 26, slice | (W - 1) << 13 | (H - 1) << 18}.
 struct RasterScratch {
   unsigned long long *keys;  // width * height
@@ -536,7 +537,7 @@ __device__ __forceinline__ void flush_quads(Collected &C, const DevCamera &cam,
     const float eye[3] = {cam.eye[0], cam.eye[1], cam.eye[2]};
     for (uint32_t q = wave; q < n; q += kQuadThreads / 64u) {
       const QuadGeom g = unpack_geom(C.geom[q].x, C.geom[q].y);
-      const uint32_t xy = C.xy[q], w = C.rw[q], a = C.area[q];
+      const uint32_t xy = C.xy[q], w = C.rw[q] & 0xFFFFu, a = C.area[q] / (C.rw[q] >> 16) * w;
       for (uint32_t p = lane; p < a; p += 64u)
         test_pixel(g, eye, (uint64_t)((xy >> 14) + p / w) * (uint32_t)cam.width + (xy & 0x3FFFu) + p % w,
                    npx, C.id[q], s);
@@ -552,8 +553,8 @@ __device__ __forceinline__ void flush_quads(Collected &C, const DevCamera &cam,
 // longer, at 6 and 8 the spills cost more than the waves gain.
 __global__ void __launch_bounds__(kQuadThreads, 5) raster_quads_kernel(
     DevCamera cam, RasterView view, const uint32_t *slot_chunk, const uint32_t *slot_count,
-    const uint32_t *quads, uint32_t per_slot, uint32_t nc, uint32_t batch, bool occlude,
-    DepthLevels depth, RasterScratch s) {
+    const uint32_t *quads, uint32_t per_slot, uint32_t nc, uint32_t batch, uint32_t spread,
+    bool occlude, DepthLevels depth, RasterScratch s) {
   __shared__ Collected C;
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -631,8 +632,9 @@ __global__ void __launch_bounds__(kQuadThreads, 5) raster_quads_kernel(
         at += (uint32_t)__popcll(lives & ((1ull << lane) - 1ull));
         C.id[at] = id;
         C.xy[at] = (uint32_t)r[0] | ((uint32_t)r[2] << 14);
-        C.rw[at] = rw;
-        C.area[at] = rw * (uint32_t)(r[3] - r[2]);
+        const uint32_t ws = tests_per_row(rw, (uint32_t)(r[3] - r[2]), spread);
+        C.rw[at] = rw | (ws << 16);
+        C.area[at] = ws * (uint32_t)(r[3] - r[2]);
         C.geom[at] = geom;
       }
       __syncthreads();
@@ -688,7 +690,7 @@ __global__ void __launch_bounds__(64) raster_pixels_kernel(DevCamera cam, Raster
       const int32_t last = __builtin_amdgcn_readlane(at, 63);
       const uint32_t stop = last < (int32_t)len ? (uint32_t)last : len;  // tests these cover
       if (at >= (int32_t)done && at < (int32_t)stop) owner_at[at] = lane + 1u;
-      const float iw = a.w ? 1.0f / (float)a.w : 0.0f;
+      const float iw = a.w ? 1.0f / (float)(a.w >> 16) : 0.0f;
       uint32_t carry = 0;
       __builtin_amdgcn_wave_barrier();
       for (uint32_t g0 = done; g0 < stop; g0 += 64u) {
@@ -712,10 +714,11 @@ __global__ void __launch_bounds__(64) raster_pixels_kernel(DevCamera cam, Raster
         const QuadGeom g = unpack_geom((uint32_t)__shfl((int)b.x, (int)own, 64),
                                        (uint32_t)__shfl((int)b.y, (int)own, 64));
         if (p < stop && ow) {
-          const uint32_t k = (uint32_t)((int32_t)p - oat), py = div_pixels(k, ow, oiw);
-          const uint64_t pix = (uint64_t)((xy >> 14) + py) * (uint32_t)cam.width +
-                               (xy & 0x3FFFu) + (k - py * ow);
-          test_pixel(g, eye, pix, npx, id, s);
+          const uint32_t k = (uint32_t)((int32_t)p - oat), ws = ow >> 16;
+          const uint32_t py = div_pixels(k, ws, oiw);
+          const uint64_t row = (uint64_t)((xy >> 14) + py) * (uint32_t)cam.width + (xy & 0x3FFFu);
+          for (uint32_t x = k - py * ws; x < (ow & 0xFFFFu); x += ws)
+            test_pixel(g, eye, row + x, npx, id, s);
         }
       }
       __builtin_amdgcn_wave_barrier();
@@ -965,7 +968,7 @@ meso_status meso_raster_pool(meso_raster *r, meso_chunk_pool *pool, const meso_c
                        bound[k] * bound[k], bound[k + 1] * bound[k + 1], k > 0, depth, r->s);
     MESO_HIP(hipGetLastError());
     hipLaunchKernelGGL(raster_quads_kernel, dim3(std::min(waves / 8u, kMaxLotGroups)), dim3(kQuadThreads), 0, s, dc, v, pv.slot_chunk,
-                       pv.slot_count, pv.quads, per, (uint32_t)pv.nc, batch, k > 0, depth, r->s);
+                       pv.slot_count, pv.quads, per, (uint32_t)pv.nc, batch, test_spread(npx), k > 0, depth, r->s);
     MESO_HIP(hipGetLastError());
     hipLaunchKernelGGL(raster_pixels_kernel, dim3(2u * waves), dim3(64), 0, s, dc, r->s);
     MESO_HIP(hipGetLastError());

@@ -90,3 +90,21 @@ def test_listed_quads(ctx, pools):
                         st["slot_count"], st["quads"], 16384, O.shading(W.LIGHT).light)
     top = ref[0][ref[1] == 2]  # +y hits: of the four 32x32 floor quads at least one is so large
     assert len(top) // 4 > 4 * 256
+
+
+# quads of more pixels than a quad has tests, and a frame above the 2^26 pixels
+# up to which a test is one pixel
+@pytest.mark.parametrize("w,h", [(1920, 1080), (16384, 4097)])
+def test_quads_of_many_pixels(ctx, pools, w, h):
+    n, nc, pool, st = pools["slab"]
+    eye, target, fov = (20.3, 9.1, 6.2), (40.0, 4.0, 50.0), 70.0
+    rast, tg = R.Raster(ctx, w, h), R.RayTargets(ctx, w, h)
+    rast.draw(pool, R.camera(eye, target, UP, fov, w, h), R.shading(W.LIGHT), tg)
+    ctx.sync()
+    assert rast.stats()["overflow_quads"] == 0
+    ref = O.raster_pool(O.camera(eye, target, UP, fov, w, h), n, nc, st["slot_chunk"],
+                        st["slot_count"], st["quads"], 16384, O.shading(W.LIGHT).light)
+    assert (ref[1] == 2).sum() > 1 << 19  # the floor's few quads
+    for got, want in zip(tg.results(), ref[:4]):
+        assert np.array_equal(got.view(np.uint8), want.view(np.uint8))
+    rast.destroy()

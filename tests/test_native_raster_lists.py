@@ -1,7 +1,8 @@
 """The quad rasteriser's list counter (mesoengine_amd/csrc/raster_lists.h)
 replayed on the CPU past the capacity of its fields (2^24 records, 2^40 tests),
 in small and in very many lots: neither field wraps, and the lots that are
-listed fill the lists from their start without gaps."""
+listed fill the lists from their start without gaps.  And how a quad's pixels
+are cut into tests: each in one, and never so many that a lot is refused."""
 import os
 import subprocess
 
@@ -35,3 +36,9 @@ def test_fields_never_wrap(replay, seed, quads, groups, records, windows, area):
     r = subprocess.run([replay] + [str(v) for v in (seed, quads, groups, records, windows, area)],
                        capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("seed", [1, 2, 3])
+def test_rectangles_are_cut_into_tests(replay, seed):
+    r = subprocess.run([replay, "cut", str(seed), "4000"], capture_output=True, timeout=120)
+    assert r.returncode == 0
